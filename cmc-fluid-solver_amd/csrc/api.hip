@@ -222,12 +222,12 @@ class Solver final : public ISolver {
             for (int f = 0; f < 4; f++)
                 for (int64_t k = 0; k < N; k++) hg[f][o + k] = (T)src[f][k];
         }
-        CMCX_HIP(hipMalloc((void**)&d_type, NT));
-        CMCX_HIP(hipMalloc((void**)&d_bcv, NT));
-        CMCX_HIP(hipMalloc((void**)&d_bct, NT));
-        CMCX_HIP(hipMalloc((void**)&d_tflags, NT));
-        for (int f = 0; f < 4; f++) CMCX_HIP(hipMalloc((void**)&d_g[f], sizeof(T) * NT));
-        CMCX_HIP(hipMalloc((void**)&buf, sizeof(T) * NT * 20));
+        CMCX_HIP(hipMalloc((void**)&d_type, NT + kSlack));
+        CMCX_HIP(hipMalloc((void**)&d_bcv, NT + kSlack));
+        CMCX_HIP(hipMalloc((void**)&d_bct, NT + kSlack));
+        CMCX_HIP(hipMalloc((void**)&d_tflags, NT + kSlack));
+        for (int f = 0; f < 4; f++) CMCX_HIP(hipMalloc((void**)&d_g[f], sizeof(T) * (NT + kSlack)));
+        CMCX_HIP(hipMalloc((void**)&buf, sizeof(T) * (NT * 20 + kSlack)));
         CMCX_HIP(hipMemsetAsync(buf, 0, sizeof(T) * NT * 20, st));
         Layer4<T>* Ls[5] = {&cur, &next, &half, &tA, &tB};
         for (int l = 0; l < 5; l++)
@@ -1182,7 +1182,7 @@ class Solver final : public ISolver {
         if (need > adj.tape_layers || adj.tape_G != adj.G) {
             hipFree(adj.tape);
             adj.tape = nullptr;
-            CMCX_HIP(hipMalloc((void**)&adj.tape, sizeof(T) * 4 * NT * need));
+            CMCX_HIP(hipMalloc((void**)&adj.tape, sizeof(T) * (4 * NT * need + kSlack)));
             adj.tape_layers = need;
             adj.tape_G = adj.G;
             adj.holds[0] = adj.holds[1] = -1;
@@ -1267,7 +1267,7 @@ class Solver final : public ISolver {
         const int64_t per = 1 + 6 * (int64_t)adj.G;
         ensure_tape(false);
         if (!adj.work) {
-            CMCX_HIP(hipMalloc((void**)&adj.work, sizeof(T) * 4 * NT * 6));
+            CMCX_HIP(hipMalloc((void**)&adj.work, sizeof(T) * (4 * NT * 6 + kSlack)));
             CMCX_HIP(hipMalloc((void**)&adj.pp, sizeof(double) * 4 * adj_point_blocks()));
             CMCX_HIP(hipMalloc((void**)&adj.nmask, sizeof(uint16_t) * g.N));
             for (int a = 0; a < 3; a++)

@@ -18,6 +18,10 @@ enum { AX_X = 0, AX_Y = 1, AX_Z = 2 };
 
 void set_error(const std::string& msg);
 
+// Elements behind the end of every flat array that a sweep reads in runs along
+// z: the last run of a line may reach up to 15 elements past it.
+constexpr int64_t kSlack = 16;
+
 struct HipError {
     hipError_t code;
     std::string where;
@@ -111,8 +115,6 @@ struct FusedWork {
     int32_t* d_inst = nullptr;   // Z: grid of each work-group
     int maxn = 0;                // longest line along the axis over the grids
     int kmax = 1;                // X/Y: tiles per work item
-    int vec_ok = 1;              // Z: every line starts on a 16-byte boundary
-    int nz_gcd = 0;              // Z: greatest common divisor of the grids' nz
     int stream = 0;              // sweeps store past the caches (kStoreStream)
     void release();
 };

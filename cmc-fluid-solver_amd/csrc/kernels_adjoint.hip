@@ -217,7 +217,7 @@ __global__ void __launch_bounds__(MAXT) adj_solve_kernel(
 // accesses), two lines per wavefront, kZWaves wavefronts per work-group.  The
 // coefficients of the rows either side of a chunk come from the neighbouring
 // lanes by shuffle (c of the previous row, a of the next row).
-template <class T, int M, bool VALL>
+template <class T, int M>
 __global__ void __launch_bounds__(64 * kZWaves) adj_z_kernel(
     Geom g, SweepParams<T> p, const uint8_t* __restrict__ type, const uint8_t* __restrict__ bcv,
     const uint8_t* __restrict__ bct, Layer4<T> tin, Layer4<T> xs, T xscale, Layer4<T> tb, T beta,
@@ -235,7 +235,7 @@ __global__ void __launch_bounds__(64 * kZWaves) adj_z_kernel(
     const int r0 = ll * M;
     const bool ok = live && ll < used;
     const int valid = ok ? min(M, n - r0) : 0;
-    const bool vec = VALL && valid == M;
+    const bool whole = valid == M;
     const int64_t c0 = base + r0;
 
     // Every load of the lane goes out in one batch (a value used under a
@@ -243,21 +243,21 @@ __global__ void __launch_bounds__(64 * kZWaves) adj_z_kernel(
     // kinds, the advecting velocity, xbar, tbar and the accumulator of the
     // lane's rows; the raw values are then used once, all together.
     int tyr[M], bvr[M], btr[M];
-    load_bytes_raw<M, VALL>(type, c0, valid, tyr);
-    load_bytes_raw<M, VALL>(bcv, c0, valid, bvr);
-    load_bytes_raw<M, VALL>(bct, c0, valid, btr);
+    load_bytes<M>(type, c0, ok, tyr);
+    load_bytes<M>(bcv, c0, ok, bvr);
+    load_bytes<M>(bct, c0, ok, btr);
     T w[M];
-    load_run_raw<T, M, VALL>(tin.f[2], c0, valid, w);
+    load_run<T, M>(tin.f[2], c0, ok, w);
     const bool hasx = xs.f[0] != nullptr;  // xbar = xscale * xs, or zero
     T xa[4][M], ta[4][M], ca[4][M];
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-        load_run_raw<T, M, VALL>(hasx ? xs.f[v] : tb.f[v], c0, valid, xa[v]);
-        load_run_raw<T, M, VALL>(tb.f[v], c0, valid, ta[v]);
+        load_run<T, M>(hasx ? xs.f[v] : tb.f[v], c0, ok, xa[v]);
+        load_run<T, M>(tb.f[v], c0, ok, ta[v]);
         // the state adjoint's accumulator (the input of a Z sweep is the
         // state): (3/dt) lam is added to it on NODE_IN rows (zacc 2) or
         // starts it (zacc 1)
-        load_run_raw<T, M, VALL>(zacc == 2 ? cacc.f[v] : tb.f[v], c0, valid, ca[v]);
+        load_run<T, M>(zacc == 2 ? cacc.f[v] : tb.f[v], c0, ok, ca[v]);
     }
 #pragma unroll
     for (int j = 0; j < M; j++) {
@@ -345,12 +345,12 @@ __global__ void __launch_bounds__(64 * kZWaves) adj_z_kernel(
                 x[j] = ch.E[v][j] + F * xf[v] + G * xl[v];
             }
         }
-        store_run<T, M>(lam.f[v] + c0, x, vec, valid);
+        store_run<T, M>(lam.f[v] + c0, x, whole, valid);
         if (zacc) {
 #pragma unroll
             for (int j = 0; j < M; j++)
                 if (role[j] == RL_IN) ca[v][j] = zacc == 2 ? ca[v][j] + p.three_dt * x[j] : p.three_dt * x[j];
-            store_run<T, M>(cacc.f[v] + c0, ca[v], vec, valid);
+            store_run<T, M>(cacc.f[v] + c0, ca[v], whole, valid);
         }
     }
 }
@@ -741,21 +741,13 @@ void launch_adj_sweep(const Geom& g, int axis, const SweepParams<T>& p, const ui
         if (ntiles > 0) {
             const int m = adj_z_chunk(g.nz);
             const size_t lds = 0;
-            // whole 16-byte aligned runs: every lane's M rows inside its line
-            const int vec_ok = ((size_t)g.nz * sizeof(T)) % 16 == 0 && g.nz % m == 0 ? 1 : 0;
-#define LZ(MM, VA)                                                                              \
-    hipLaunchKernelGGL((adj_z_kernel<T, MM, VA>), dim3((unsigned)ntiles), dim3(64 * kZWaves), lds, \
-                       st, g, p, type, bcv, bct, tin, xs, xscale, tb, beta, lam, cacc,             \
+#define LZ(MM)                                                                                  \
+    hipLaunchKernelGGL((adj_z_kernel<T, MM>), dim3((unsigned)ntiles), dim3(64 * kZWaves), lds, st, \
+                       g, p, type, bcv, bct, tin, xs, xscale, tb, beta, lam, cacc,                 \
                        zmode ? (first_z ? 1 : 2) : 0, tiles)
-            if (vec_ok) {
-                if (m == 2) LZ(2, true);
-                else if (m == 4) LZ(4, true);
-                else LZ(8, true);
-            } else {
-                if (m == 2) LZ(2, false);
-                else if (m == 4) LZ(4, false);
-                else LZ(8, false);
-            }
+            if (m == 2) LZ(2);
+            else if (m == 4) LZ(4);
+            else LZ(8);
 #undef LZ
             CMCX_LAUNCH_CHECK();
         }

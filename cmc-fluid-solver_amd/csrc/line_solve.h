@@ -456,51 +456,17 @@ struct Vec16<double> {
     static constexpr int n = 2;
 };
 
-// r[0..M) <- p[0..M): 16-byte loads when `vec` (all M rows inside the line and
-// aligned), else element loads of the first `valid` rows (zero beyond).
+// Vector of W consecutive elements at any element address: global vector loads
+// and stores need no more than element alignment on this architecture
+// (unaligned access mode), so a run that starts anywhere in memory is read and
+// written 16 bytes at a time like an aligned one.
+template <class T, int W>
+struct RunVec {
+    typedef T type __attribute__((ext_vector_type(W), aligned(sizeof(T))));
+};
+// elements per vector of a run of M rows
 template <class T, int M>
-__device__ __forceinline__ void load_run(const T* __restrict__ p, T* r, bool vec, int valid) {
-    constexpr int VW = Vec16<T>::n;
-    if constexpr (M % VW == 0) {
-        if (vec) {
-            using V = typename Vec16<T>::type;
-#pragma unroll
-            for (int k = 0; k < M / VW; k++) {
-                V v = reinterpret_cast<const V*>(p)[k];
-                const T* e = reinterpret_cast<const T*>(&v);
-#pragma unroll
-                for (int q = 0; q < VW; q++) r[k * VW + q] = e[q];
-            }
-            return;
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < M; j++) r[j] = j < valid ? p[j] : (T)0;
-}
-
-// r[0..M) <- bytes p[0..M): one M-byte load when `vec` and p is M-byte aligned
-// (M = 2, 4, 8, 16), else byte loads of the first `valid` bytes (zero beyond).
-template <int M>
-__device__ __forceinline__ void load_bytes(const uint8_t* __restrict__ p, uint8_t* r, bool vec,
-                                           int valid) {
-    if (vec && ((uintptr_t)p % M) == 0) {
-        if constexpr (M == 2) {
-            const uint16_t w = *reinterpret_cast<const uint16_t*>(p);
-            r[0] = (uint8_t)w; r[1] = (uint8_t)(w >> 8);
-            return;
-        } else if constexpr (M == 4 || M == 8 || M == 16) {
-            using W = typename std::conditional<M == 4, uint32_t,
-                      typename std::conditional<M == 8, uint2, uint4>::type>::type;
-            const W w = *reinterpret_cast<const W*>(p);
-            const uint8_t* b = reinterpret_cast<const uint8_t*>(&w);
-#pragma unroll
-            for (int j = 0; j < M; j++) r[j] = b[j];
-            return;
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < M; j++) r[j] = j < valid ? p[j] : (uint8_t)0;
-}
+constexpr int run_width() { return M < Vec16<T>::n ? M : Vec16<T>::n; }
 
 // A store with a cache hint: NT streams it past the caches (non-temporal),
 // for sweeps whose layers far exceed the memory-side cache, where written
@@ -511,21 +477,20 @@ __device__ __forceinline__ void put_hint(T* p, T v) {
     else *p = v;
 }
 
+// p[0..M) <- r when `whole`, else its first `valid` rows.
 template <class T, int M, bool NT = false>
-__device__ __forceinline__ void store_run(T* __restrict__ p, const T* r, bool vec, int valid) {
-    constexpr int VW = Vec16<T>::n;
-    if constexpr (M % VW == 0) {
-        if (vec) {
-            typedef T NV __attribute__((ext_vector_type(VW)));
+__device__ __forceinline__ void store_run(T* __restrict__ p, const T* r, bool whole, int valid) {
+    constexpr int VW = run_width<T, M>();
+    using NV = typename RunVec<T, VW>::type;
+    if (whole) {
 #pragma unroll
-            for (int k = 0; k < M / VW; k++) {
-                NV v;
+        for (int k = 0; k < M / VW; k++) {
+            NV v;
 #pragma unroll
-                for (int q = 0; q < VW; q++) v[q] = r[k * VW + q];
-                put_hint<NT>(reinterpret_cast<NV*>(p) + k, v);
-            }
-            return;
+            for (int q = 0; q < VW; q++) v[q] = r[k * VW + q];
+            put_hint<NT>(reinterpret_cast<NV*>(p + k * VW), v);
         }
+        return;
     }
 #pragma unroll
     for (int j = 0; j < M; j++)
@@ -547,48 +512,36 @@ __device__ __forceinline__ void with_store_hint(bool nt, F&& f) {
     }
 }
 
-// Loads of one lane's run of M rows at c0 (the first `valid` of them inside
-// the line), all issued whatever `valid` is: rows past it read from node 0
-// (addresses masked, not selected, so that no load becomes conditional).
-// `vall`: every run of the launch is whole and 16-byte aligned (vector loads).
-template <class T, int M, bool VALL>
-__device__ __forceinline__ void load_run_raw(const T* __restrict__ p, int64_t c0, int valid, T* r) {
-    constexpr int VW = Vec16<T>::n;
-    if constexpr (M % VW == 0 && VALL) {
-        {
-            using V = typename Vec16<T>::type;
-            const V* q = reinterpret_cast<const V*>(p + (c0 & -(int64_t)(valid > 0)));
+// Loads of one lane's run of M rows at c0, all issued whatever the number of
+// rows inside the line (a lane without rows reads node 0: its address is
+// masked, not selected, so that no load becomes conditional).  The last run of
+// a line may reach up to M - 1 rows past the line's end; the values read there
+// are the next line's (or the arrays' slack, kSlack elements) and are not used.
+template <class T, int M>
+__device__ __forceinline__ void load_run(const T* __restrict__ p, int64_t c0, bool any, T* r) {
+    constexpr int VW = run_width<T, M>();
+    using V = typename RunVec<T, VW>::type;
+    const T* q = p + (c0 & -(int64_t)any);
 #pragma unroll
-            for (int k = 0; k < M / VW; k++) {
-                const V v = q[k];
-                const T* e = reinterpret_cast<const T*>(&v);
+    for (int k = 0; k < M / VW; k++) {
+        const V v = *reinterpret_cast<const V*>(q + k * VW);
 #pragma unroll
-                for (int i = 0; i < VW; i++) r[k * VW + i] = e[i];
-            }
-            return;
-        }
+        for (int i = 0; i < VW; i++) r[k * VW + i] = v[i];
     }
-#pragma unroll
-    for (int j = 0; j < M; j++) r[j] = p[(c0 + j) & -(int64_t)(j < valid)];
 }
 
-template <int M, bool VALL>
-__device__ __forceinline__ void load_bytes_raw(const uint8_t* __restrict__ p, int64_t c0, int valid,
-                                               int* r) {
-    if constexpr ((M == 4 || M == 8) && VALL) {
-        {
-            const uint32_t* q = reinterpret_cast<const uint32_t*>(p + (c0 & -(int64_t)(valid > 0)));
+// The same for a run of M bytes.
+template <int M>
+__device__ __forceinline__ void load_bytes(const uint8_t* __restrict__ p, int64_t c0, bool any, int* r) {
+    constexpr int W = M < 4 ? M : 4;
+    const uint8_t* q = p + (c0 & -(int64_t)any);
 #pragma unroll
-            for (int k = 0; k < M / 4; k++) {
-                const uint32_t v = q[k];
+    for (int k = 0; k < M / W; k++) {
+        uint32_t v = 0;
+        __builtin_memcpy(&v, q + k * W, W);
 #pragma unroll
-                for (int i = 0; i < 4; i++) r[4 * k + i] = (v >> (8 * i)) & 0xff;
-            }
-            return;
-        }
+        for (int i = 0; i < W; i++) r[W * k + i] = (v >> (8 * i)) & 0xff;
     }
-#pragma unroll
-    for (int j = 0; j < M; j++) r[j] = p[(c0 + j) & -(int64_t)(j < valid)];
 }
 
 template <class T>
