@@ -121,10 +121,15 @@ struct FusedWork {
 
 // Stores bit of the fused sweeps: non-temporal stores of the output and the
 // merged Picard layer.  Set for launches whose 16 fields moved per sweep
-// exceed kStreamStoreBytes, the MI355X memory-side cache (256 MiB).  Measured
-// on the ellipsoids workload, FP32, step time with streamed against plain
-// stores: 128^3 (134 MB per sweep, which the cache holds) +14 %, 160^3
-// (262 MB) -0.8 %, 192^3 (453 MB) -6.2 %, 256^3 (1.07 GB) -8 to -10 %.
+// exceed kStreamStoreBytes, the MI355X memory-side cache (256 MiB), and whose z
+// lines are whole 128-byte cache lines.  Measured on the ellipsoids workload,
+// FP32, step time with streamed against plain stores: 128^3 (134 MB per sweep,
+// which the cache holds) +14 %, 160^3 (262 MB) -0.8 %, 192^3 (453 MB) -6.2 %,
+// 256^3 (1.07 GB) -8 to -10 %.  Rows that start anywhere leave partial lines at
+// both ends, which only plain stores can merge with the neighbour tile's in
+// the caches: a 250 x 203 x 187 grid takes X 177, Y 204, Z 157 us per sweep
+// with plain and 193, 306, 172 with streamed stores; with lines of a multiple
+// of 64 bytes (240^3, 208^3) the two are level.
 constexpr int kStoreStream = 4;
 constexpr int64_t kStreamStoreBytes = 256ll << 20;
 

@@ -794,6 +794,11 @@ void launch_fused_sweep(const InstDesc<T>* insts, T three_dt, int axis, const Fu
         if (m == 0) throw std::string("fused sweep: Z variant does not fit the line length");
         const int vw = 16 / (int)sizeof(T);
         const int nthreads = 64 * kZWaves * (lpl / 32);
+        // a lane's run of more than one 16-byte vector leaves partial lines
+        // after each store instruction: streamed, they cost 5 to 40 % (256^2
+        // planes: FP32 lines of 256 in 8 rows per lane 200 -> 219 us, FP64 in
+        // 8 rows 336 -> 464, in 4 rows 242 -> 253)
+        if (m * (int)sizeof(T) > 16) stores &= ~kStoreStream;
         const size_t lds = park ? (size_t)(nthreads / 64) * 64 * 4 * ((m + vw - 1) / vw) * 16 : 0;
 #define LZ(MM, W, PK, LL)                                                                         \
     hipLaunchKernelGGL((fused_z_kernel<T, MM, W, PK, LL>), dim3(blocks), dim3(nthreads), lds, st, \
@@ -901,10 +906,15 @@ void build_fused_work(const uint8_t* h_type, const std::vector<Geom>& geoms,
     std::vector<int32_t> items, winst;
     {
         // stream the stores of sweeps whose fields exceed the memory-side
-        // cache (16 fields move per sweep)
+        // cache (16 fields move per sweep), if every z line is whole cache
+        // lines (see kStreamStoreBytes)
         int64_t cells = 0;
-        for (const Geom& g : geoms) cells += (int64_t)g.nx * g.ny * g.nz;
-        w.stream = (double)cells * (double)elem * 16.0 > (double)kStreamStoreBytes ? 1 : 0;
+        bool whole = true;
+        for (const Geom& g : geoms) {
+            cells += (int64_t)g.nx * g.ny * g.nz;
+            whole = whole && (size_t)g.nz * elem % 128 == 0;
+        }
+        w.stream = whole && (double)cells * (double)elem * 16.0 > (double)kStreamStoreBytes ? 1 : 0;
     }
     w.maxn = 0;
     w.kmax = 1;

@@ -488,7 +488,9 @@ __device__ __forceinline__ void store_run(T* __restrict__ p, const T* r, bool wh
             NV v;
 #pragma unroll
             for (int q = 0; q < VW; q++) v[q] = r[k * VW + q];
-            put_hint<NT>(reinterpret_cast<NV*>(p + k * VW), v);
+            NV* const q = reinterpret_cast<NV*>(p + k * VW);  // element-aligned
+            if constexpr (NT) __builtin_nontemporal_store(v, q);
+            else *q = v;
         }
         return;
     }
