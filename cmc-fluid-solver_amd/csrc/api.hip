@@ -564,6 +564,10 @@ class Solver final : public ISolver {
         p.inv_2hx = (T)1 / (2 * p.hx);
         p.inv_2hy = (T)1 / (2 * p.hy);
         p.inv_2hz = (T)1 / (2 * p.hz);
+        p.kp = p.v_T * p.inv_2h;
+        p.kd = p.t_phi * p.inv_2h * p.inv_2h;
+        p.ka = p.t_phi * p.inv_2h * (axis == AX_X ? p.inv_2hy : p.inv_2hx);
+        p.kb = p.t_phi * p.inv_2h * (axis == AX_Z ? p.inv_2hy : p.inv_2hz);
         return p;
     }
 

@@ -68,6 +68,9 @@ struct SweepParams {
     T three_dt;   // 3 / dt
     T inv_2h;     // 1 / (2 h)
     T inv_2hx, inv_2hy, inv_2hz;
+    // products of the fused rows: v_T / 2h, t_phi / (2h)^2 and t_phi / (2h 2h_o)
+    // for the two other axes o in x, y, z order
+    T kp, kd, ka, kb;
 };
 
 template <class T>

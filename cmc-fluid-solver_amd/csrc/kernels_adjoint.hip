@@ -89,7 +89,6 @@ __global__ void __launch_bounds__(MAXT) adj_solve_kernel(
     const int gl = lane % LPG;
     const int chunk = wave * GPW + lane / LPG;
     const int P = nw * GPW;
-    const RedLayout L{2 * P, kRedFields * 2 * P + 1};
 
     const int tile = tiles[xcd_remap(blockIdx.x, gridDim.x)];
     const int outer = tile / ltiles;
@@ -173,25 +172,13 @@ __global__ void __launch_bounds__(MAXT) adj_solve_kernel(
         c0 = cp;
     }
     if (M >= 3) chunk_up<T, M>(ch);
+    T xf[4], xl[4];
     {
         T f[kRedFields], l[kRedFields];
         chunk_reduced<T, M>(ch, rfirst, rlast, f, l);
-#pragma unroll
-        for (int k = 0; k < kRedFields; k++) {
-            red[L.at(gl, k, 2 * chunk)] = f[k];
-            red[L.at(gl, k, 2 * chunk + 1)] = l[k];
-        }
+        chunk_ends<T>(red, gl, LPG, chunk, P, wave, nw, f, l, xf, xl);
     }
-    __syncthreads();
-    solve_reduced_compact<T>(red, L, LPG, wave, nw);
-    __syncthreads();
     if (!ok) return;
-    T xf[4], xl[4];
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-        xf[v] = red[L.at(gl, 6 + v, 2 * chunk)];
-        xl[v] = red[L.at(gl, 6 + v, 2 * chunk + 1)];
-    }
 #pragma unroll
     for (int j = 0; j < M; j++) {
         const int rl = role[j + 1];
@@ -765,7 +752,7 @@ void launch_adj_sweep(const Geom& g, int axis, const SweepParams<T>& p, const ui
             waves++;
         }
         const int P = waves * (64 / lpg);
-        const size_t lds = (size_t)lpg * (kRedFields * 2 * P + 1) * sizeof(T);
+        const size_t lds = (size_t)ends_elems(lpg, P) * sizeof(T);
 #define LA(AX, LPG)                                                                               \
     hipLaunchKernelGGL((adj_solve_kernel<T, AX, kAdjChunk, LPG, 512>), dim3((unsigned)ntiles),    \
                        dim3(64 * waves), lds, st, g, p, type, bcv, bct, tin, xs, xscale, tb, beta, lam, \

@@ -30,9 +30,23 @@
 //
 // Each line is solved by the chunked partition method of line_solve.h (chunks
 // of M rows per lane, reduced system of 2 rows per chunk, compacted by one
-// cyclic-reduction step to one row per chunk, at most 32 rows per line, then
-// PCR across the lanes: through LDS for strided lines, in registers for Z).  The U, V and W systems share one matrix (same
-// bc_vel and viscosity); T has its own.
+// cyclic-reduction step to one row per chunk, then PCR across the lanes until
+// the rows are decoupled: through LDS for strided lines, in registers for Z).
+// The U, V and W systems share one matrix (same bc_vel and viscosity); T has
+// its own.
+//
+// Instructions.  Four wavefronts per SIMD leave the sweeps bound by the vector
+// instructions they issue as much as by memory (SQ counters: 18 % of a
+// wavefront's time issuing, 45-49 % waiting to), and on small grids a lone
+// wavefront's instruction stream is most of the sweep.  So a row costs about a
+// hundred of them: boundary handling is left out where no row of the wavefront
+// needs it (bit_role), one 32-bit byte offset per row serves every field
+// (at_byte), the stores' switches are outside the row loops, and the dissipation
+// takes its differences from the advection term.  With the rows handled one by
+// one, selects for every role and a 64-bit address per access (over 300 per
+// row) the sweeps took, X / Y / Z in us: 32^3 FP32 9.3 / 9.9 / 5.0, now 6.6 /
+// 7.5 / 3.8; 64^3 11.2 / 12.3 / 9.2, now 8.3 / 10.5 / 7.6; 250 x 203 x 187 167
+// / 202 / 142, now 152 / 190 / 142; 256^3 267 / 303 / 187, now 261 / 272 / 185.
 //
 // Node flags: the fused kernels read one byte per node, the node type in bits
 // 0-1 and the BC kinds (BC_FREE) of velocity and T in bits 2 and 3 (0 for
@@ -87,43 +101,71 @@ using namespace lsolve;
 // before, at and after the node (per field), cin the sweep input at the node,
 // ca and cb the central differences (not yet scaled) of the cross-line
 // derivatives of Phi_d (X: u along y and z; Y: v along x and z; Z: w along x
-// and y) (TimeLayer3D.h:338-343, 554-588).
+// and y) (TimeLayer3D.h:338-343, 554-588).  With D f = f(+1) - f(-1) along the
+// sweep and a its velocity component, t_phi Phi_d is
+//   kd (sum of (D f)^2 over u, v, w, once more for a)
+//   + ka D f1 ca + kb D f2 cb,  f1, f2 the components along ca and cb.
+// b is the same on every interior row (bv, bt).
 template <class T, int AXIS>
-__device__ __forceinline__ void interior_row_delta(const SweepParams<T>& p, const T* wm,
+__device__ __forceinline__ void interior_row_delta(const SweepParams<T>& p, T bv, T bt, const T* wm,
                                                    const T* w0, const T* wp, const T* cin, T ca,
                                                    T cb, Row<T>& r) {
+    constexpr int F1 = AXIS == AX_X ? 1 : 0, F2 = AXIS == AX_Z ? 1 : 2;
     const T adv = w0[AXIS] * p.inv_2h;
     r.av = -adv - p.vis_v;
     r.cv = adv - p.vis_v;
-    r.bv = p.three_dt + 2 * p.vis_v;
+    r.bv = bv;
     r.at = -adv - p.vis_t;
     r.ct = adv - p.vis_t;
-    r.bt = p.three_dt + 2 * p.vis_t;
+    r.bt = bt;
+    T df[4];
 #pragma unroll
     for (int v = 0; v < 4; v++) {
         const T vis = v < 3 ? p.vis_v : p.vis_t;
-        r.d[v] = p.three_dt * (cin[v] - w0[v]) + adv * (wm[v] - wp[v]) +
-                 vis * ((wm[v] + wp[v]) - 2 * w0[v]);
+        df[v] = wp[v] - wm[v];
+        r.d[v] = p.three_dt * (cin[v] - w0[v]) - adv * df[v] + vis * ((wm[v] + wp[v]) - 2 * w0[v]);
     }
-    r.d[AXIS] = r.d[AXIS] - p.v_T * ((wp[3] - wm[3]) * p.inv_2h);
-    T phi;
-    if (AXIS == AX_X) {
-        const T u_x = (wp[0] - wm[0]) * p.inv_2hx, v_x = (wp[1] - wm[1]) * p.inv_2hx;
-        const T w_x = (wp[2] - wm[2]) * p.inv_2hx;
-        const T u_y = ca * p.inv_2hy, u_z = cb * p.inv_2hz;
-        phi = 2 * u_x * u_x + v_x * v_x + w_x * w_x + v_x * u_y + w_x * u_z;
-    } else if (AXIS == AX_Y) {
-        const T u_y = (wp[0] - wm[0]) * p.inv_2hy, v_y = (wp[1] - wm[1]) * p.inv_2hy;
-        const T w_y = (wp[2] - wm[2]) * p.inv_2hy;
-        const T v_x = ca * p.inv_2hx, v_z = cb * p.inv_2hz;
-        phi = u_y * u_y + 2 * v_y * v_y + w_y * w_y + u_y * v_x + w_y * v_z;
-    } else {
-        const T u_z = (wp[0] - wm[0]) * p.inv_2hz, v_z = (wp[1] - wm[1]) * p.inv_2hz;
-        const T w_z = (wp[2] - wm[2]) * p.inv_2hz;
-        const T w_x = ca * p.inv_2hx, w_y = cb * p.inv_2hy;
-        phi = u_z * u_z + v_z * v_z + 2 * w_z * w_z + u_z * w_x + v_z * w_y;
-    }
-    r.d[3] = r.d[3] + p.t_phi * phi;
+    r.d[AXIS] = r.d[AXIS] - p.kp * df[3];
+    T sq = df[AXIS] * df[AXIS];
+#pragma unroll
+    for (int v = 0; v < 3; v++) sq = sq + df[v] * df[v];
+    r.d[3] = r.d[3] + p.kd * sq + df[F1] * (p.ka * ca) + df[F2] * (p.kb * cb);
+}
+
+// Rows of a chunk as bits: bit i of `nin` is set when window row i (line row
+// r0 - 1 + i) is not NODE_IN.  The row roles follow from a row's bit and its
+// neighbours' (row_role); most rows are NODE_IN and most others hold a value
+// that the Picard layer already has, so the kernels test these bits for a whole
+// wavefront and leave out what none of its rows needs.
+__device__ __forceinline__ int bit_role(uint32_t nin, int j) {
+    const bool in = !((nin >> (j + 1)) & 1), L = !((nin >> j) & 1), R = !((nin >> (j + 2)) & 1);
+    return in ? RL_IN : L && R ? RL_SHARED : R ? RL_START : L ? RL_END : RL_NONE;
+}
+// rows of a system (role other than RL_NONE), bit i for window row i
+__device__ __forceinline__ uint32_t system_rows(uint32_t nin) {
+    const uint32_t in = ~nin;
+    return in | (in << 1) | (in >> 1);
+}
+
+// r of a NODE_IN row, else the identity row (x = 0) of a row that keeps its
+// Picard value.
+template <class T>
+__device__ __forceinline__ void keep_or_identity(bool in, Row<T>& r) {
+    r.av = in ? r.av : (T)0; r.bv = in ? r.bv : (T)1; r.cv = in ? r.cv : (T)0;
+    r.at = in ? r.at : (T)0; r.bt = in ? r.bt : (T)1; r.ct = in ? r.ct : (T)0;
+#pragma unroll
+    for (int v = 0; v < 4; v++) r.d[v] = in ? r.d[v] : (T)0;
+}
+
+// A value that is the same in every lane, as a scalar.
+__device__ __forceinline__ float uniform(float x) {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x)));
+}
+__device__ __forceinline__ double uniform(double x) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
 // Boundary or identity row (ApplyBC0 / ApplyBC1, AdiSolver3D.cpp:804-852) in
@@ -155,95 +197,124 @@ __device__ __forceinline__ bool dirichlet_row(int role, uint8_t tf, int q) {
     return role != RL_NONE && role != RL_IN && !((role == RL_START || role == RL_END) && (tf & fb));
 }
 
+// Element at a byte offset from a uniform base: one 32-bit offset register per
+// row serves every field (a grid of the fused path holds at most 256 x 256 x 512
+// nodes, so offsets within it fit).
+template <class T>
+__device__ __forceinline__ const T& at_byte(const T* base, int off) {
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + (uint32_t)off);
+}
+template <class T>
+__device__ __forceinline__ T* ptr_byte(T* base, int off) {
+    return reinterpret_cast<T*>(reinterpret_cast<char*>(base) + (uint32_t)off);
+}
+
+// A lane's rows of a strided line: byte offsets (in the field type) of row 0 and
+// of the last row of the line, of the chunk's first row, and the row stride.  A
+// row outside the line reads the line's first or last row instead, a face node,
+// not NODE_IN, and so an identity row as it should be; a lane without a line
+// reads the face node (1, 0, 1) on every row.  Every load is then unconditional
+// and in bounds, the cross-line neighbours included.
+struct RowSpan {
+    int lo, hi, first, step;
+    __device__ __forceinline__ int at(int j) const { return min(max(first + j * step, lo), hi); }
+};
+
 // Strided chunk: loads the chunk's rows (and the Picard layer one row either
-// side), eliminates them and returns the two reduced rows.  Row r of the line
-// lives at element base + r * s; rows outside [0, n), and every row when !ok,
-// read the interior node `safe` instead (so that each load is unconditional
-// and in bounds) and are identity rows.  The loads are software-pipelined:
-// those of row j + LA are issued before row j is eliminated, in one basic
-// block, so that LA + 1 rows are in flight instead of one (a row whose loads
-// sit in a branch of its own waits for all of them before the next row's
-// loads can issue).  role[] receives the row roles.  KEEP parks the chunk's
-// Picard layer in LDS for the write phase.
+// side), eliminates them and returns the two reduced rows.  The loads are
+// software-pipelined: those of row j + LA are issued before row j is
+// eliminated, so that LA + 1 rows are in flight.  `nin` receives the row bits,
+// `mixed` whether some row of the wavefront is not NODE_IN.  KEEP parks the
+// chunk's Picard layer in LDS for the write phase.
 template <class T, int AXIS, int M, bool KEEP, bool BSYNC>
-__device__ __forceinline__ void strided_chunk(const Geom& g, const SweepParams<T>& p,
+__device__ __forceinline__ void strided_chunk(const SweepParams<T>& p, T bv, T bt,
                                               const uint8_t* __restrict__ type,
                                               const T* const* gval, const Layer4<T>& in,
-                                              const Layer4<T>& tin, int base, int s, int safe,
-                                              int r0, int n, bool ok, int* role, Chunk<T, M>& ch,
-                                              T* f, T* l, T* keep, int kfs, int krs) {
+                                              const Layer4<T>& tin, const RowSpan& rs, int sa,
+                                              uint32_t& nin, bool& mixed, Chunk<T, M>& ch, T* f,
+                                              T* l, T* keep, int kfs, int krs) {
     constexpr int LA = 2;  // rows loaded ahead of the elimination
-    auto addr = [&](int i) {  // element of window row i (line row r0 - 1 + i)
-        const int r = r0 + i - 1;
-        return (ok && r >= 0 && r < n) ? base + r * s : safe;
-    };
-    auto valid = [&](int i) {
-        const int r = r0 + i - 1;
-        return ok && r >= 0 && r < n;
-    };
-    uint8_t ty[M + 2];
-#pragma unroll
-    for (int i = 0; i < M + 2; i++) {
-        const uint8_t t = type[addr(i)];
-        ty[i] = valid(i) ? t : kOutside;
-    }
     constexpr int XF = AXIS == AX_X ? 0 : 1;  // field of the cross-line derivatives
-    const int sa = AXIS == AX_X ? (int)g.sy : (int)g.sx;
-    const T* xfp = tin.f[XF];
-    // Picard layer window (rows r0-1 .. r0+M), sweep input and cross-line
+    // node flags: 0 on NODE_IN nodes
+    uint32_t tf[M + 2];
+#pragma unroll
+    for (int i = 0; i < M + 2; i++) tf[i] = type[(uint32_t)rs.at(i - 1) / (uint32_t)sizeof(T)];
+    // Picard layer window (rows -1 .. M), sweep input and cross-line
     // differences, filled LA rows ahead of their use
     T w[4][M + 2], cin[4][M], ca[M], cb[M];
     auto load_row = [&](int j) {  // window row j + 1 and row j's own values
-        const int c = addr(j + 1);
+        const int c = rs.at(j);
+        T e0 = 0, e2 = 0;
 #pragma unroll
-        for (int v = 0; v < 4; v++) w[v][j + 1] = tin.f[v][c];
+        for (int v = 0; v < 4; v++) {
+            const T* q = &at_byte(tin.f[v], c);
+            w[v][j + 1] = q[0];
+            if (v == XF) {
+                e0 = q[-1];
+                e2 = q[1];
+            }
+        }
 #pragma unroll
-        for (int v = 0; v < 4; v++) cin[v][j] = in.f[v][c];
-        ca[j] = xfp[c + sa] - xfp[c - sa];
-        cb[j] = xfp[c + 1] - xfp[c - 1];
+        for (int v = 0; v < 4; v++) cin[v][j] = at_byte(in.f[v], c);
+        ca[j] = at_byte(tin.f[XF], c + sa) - at_byte(tin.f[XF], c - sa);
+        cb[j] = e2 - e0;
     };
-    {
-        const int c = addr(0);
+    auto load_edge = [&](int j) {
+        const int c = rs.at(j);
 #pragma unroll
-        for (int v = 0; v < 4; v++) w[v][0] = tin.f[v][c];
-    }
+        for (int v = 0; v < 4; v++) w[v][j + 1] = at_byte(tin.f[v], c);
+    };
+    load_edge(-1);
 #pragma unroll
     for (int j = 0; j < LA && j < M; j++) load_row(j);
+    nin = 0;
+    uint32_t any = 0;
 #pragma unroll
-    for (int j = 0; j < M; j++) role[j] = row_role(ty[j + 1], ty[j], ty[j + 2]);
+    for (int i = 0; i < M + 2; i++) {
+        nin |= min(tf[i], 1u) << i;
+        any |= tf[i];
+    }
+    mixed = !__all((nin & (((1u << M) - 1) << 1)) == 0);
+    // rows with a value of their own: free ends, and every boundary row when the
+    // state is out of sync with the node values
+    const bool special = mixed && (!BSYNC || __any((any & (kFlagFreeVel | kFlagFreeT)) != 0));
     Row<T> rfirst, rlast;
 #pragma unroll
     for (int j = 0; j < M; j++) {
         if (j + LA < M) load_row(j + LA);
-        if (j + LA == M - 1 + 1 || (j == M - 1 && LA == 0)) {
-            const int c = addr(M + 1);
-#pragma unroll
-            for (int v = 0; v < 4; v++) w[v][M + 1] = tin.f[v][c];
-        }
-        T wm[4], w0[4], wp[4], ci[4], gd[4];
+        if (j + LA == M) load_edge(M);
+        T wm[4], w0[4], wp[4], ci[4];
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             wm[v] = w[v][j];
             w0[v] = w[v][j + 1];
             wp[v] = w[v][j + 2];
             ci[v] = cin[v][j];
-            gd[v] = BSYNC ? w0[v] : gval[v][addr(j + 1)];
         }
         if (KEEP) {
 #pragma unroll
             for (int v = 0; v < 4; v++) keep[v * kfs + j * krs] = w0[v];
         }
-        Row<T> ri, rb, rw;
-        interior_row_delta<T, AXIS>(p, wm, w0, wp, ci, ca[j], cb[j], ri);
-        boundary_row_delta<T>(role[j], ty[j + 1], wm, w0, wp, gd, rb);
-        const bool isin = role[j] == RL_IN;
-        rw.av = isin ? ri.av : rb.av; rw.bv = isin ? ri.bv : rb.bv; rw.cv = isin ? ri.cv : rb.cv;
-        rw.at = isin ? ri.at : rb.at; rw.bt = isin ? ri.bt : rb.bt; rw.ct = isin ? ri.ct : rb.ct;
+        Row<T> r;
+        interior_row_delta<T, AXIS>(p, bv, bt, wm, w0, wp, ci, ca[j], cb[j], r);
+        if (mixed) {
+            const bool isin = !((nin >> (j + 1)) & 1);
+            if (!special) {
+                keep_or_identity<T>(isin, r);
+            } else {
+                const int c = rs.at(j);
+                T gd[4];
 #pragma unroll
-        for (int v = 0; v < 4; v++) rw.d[v] = isin ? ri.d[v] : rb.d[v];
-        if (j == 0) rfirst = rw;
-        else if (j == M - 1) rlast = rw;
-        else chunk_down<T, M>(ch, j, rw);
+                for (int v = 0; v < 4; v++) gd[v] = BSYNC ? w0[v] : at_byte(gval[v], c);
+                Row<T> rb;
+                boundary_row_delta<T>(bit_role(nin, j), type[(uint32_t)c / (uint32_t)sizeof(T)], wm,
+                                      w0, wp, gd, rb);
+                if (!isin) r = rb;
+            }
+        }
+        if (j == 0) rfirst = r;
+        else if (j == M - 1) rlast = r;
+        else chunk_down<T, M>(ch, j, r);
         // keep the pipeline's shape: the scheduler would otherwise hoist the
         // loads of every row to the top and spill what does not fit
         __builtin_amdgcn_sched_barrier(0);
@@ -254,23 +325,22 @@ __device__ __forceinline__ void strided_chunk(const Geom& g, const SweepParams<T
 
 // Writes the chunk's rows given the corrections df / dl of its first and last
 // rows: x = t + delta on every row of a system (the node value on Dirichlet
-// rows), the merged Picard layer on NODE_IN rows.  Row j lives at element
-// base + (r0 + j) * s.  The corrections of all rows are formed first (the
-// chunk state dies there), then the Picard layer of all rows is read, then
-// everything is stored: a load issued after a store waits for the store's
-// acknowledgement as well (one counter covers both on this architecture), so
-// reads interleaved with the stores would cost a memory round trip per field.
+// rows), the merged Picard layer on NODE_IN rows.  The corrections of all rows
+// are formed first (the chunk state dies there), then the Picard layer of all
+// rows is read, then everything is stored: a load issued after a store waits
+// for the store's acknowledgement as well (one counter covers both on this
+// architecture), so reads interleaved with the stores would cost a memory round
+// trip per field.
 template <class T, int M, bool KEEP, bool BSYNC>
-__device__ __forceinline__ void strided_write(const Chunk<T, M>& ch, const int* role,
-                                              const uint8_t* __restrict__ type, int base, int s,
-                                              int safe, int r0, const T* df, const T* dl,
-                                              const T* const* gval, const Layer4<T>& tin,
-                                              const Layer4<T>& out, const Layer4<T>& tout,
-                                              int merges, int stores, const T* keep, int kfs,
-                                              int krs) {
-    // the row addresses are formed here, not kept live from the kernel's start
+__device__ __forceinline__ void strided_write(const Chunk<T, M>& ch, uint32_t nin, bool mixed,
+                                              const uint8_t* __restrict__ type, RowSpan rs,
+                                              const T* df, const T* dl, const T* const* gval,
+                                              const Layer4<T>& tin, const Layer4<T>& out,
+                                              const Layer4<T>& tout, int merges, int stores,
+                                              const T* keep, int kfs, int krs) {
+    // the row offsets are formed here, not kept live from the kernel's start
     // (where the compiler would hoist them and spill them across the solve)
-    asm volatile("" : "+v"(base), "+v"(r0), "+v"(safe));
+    asm volatile("" : "+v"(rs.first), "+v"(rs.lo), "+v"(rs.hi));
     const T km = merges > 1 ? (T)0.75 : (T)0.5;
     T dd[4][M];
 #pragma unroll
@@ -288,9 +358,9 @@ __device__ __forceinline__ void strided_write(const Chunk<T, M>& ch, const int* 
     T t0[4][M];
 #pragma unroll
     for (int j = 0; j < M; j++) {
-        const int c = role[j] != RL_NONE ? base + (r0 + j) * s : safe;
+        const int c = rs.at(j);
 #pragma unroll
-        for (int v = 0; v < 4; v++) t0[v][j] = KEEP ? keep[v * kfs + j * krs] : tin.f[v][c];
+        for (int v = 0; v < 4; v++) t0[v][j] = KEEP ? keep[v * kfs + j * krs] : at_byte(tin.f[v], c);
     }
     // every read above completes here, before the first store (otherwise the
     // compiler sinks each read into the branch of its row's stores)
@@ -298,22 +368,59 @@ __device__ __forceinline__ void strided_write(const Chunk<T, M>& ch, const int* 
     for (int j = 0; j < M; j++)
 #pragma unroll
         for (int v = 0; v < 4; v++) asm volatile("" ::"v"(t0[v][j]));
+    const uint32_t sys = system_rows(nin);
     with_store_hint((stores & kStoreStream) != 0, [&](auto ntc) {
         constexpr bool NT = decltype(ntc)::value;
+        auto put_x = [&](int j) {
+            const int c = rs.first + j * rs.step;
+            if constexpr (BSYNC) {
 #pragma unroll
-        for (int j = 0; j < M; j++) {
-            if (role[j] == RL_NONE) continue;
-            const int c = base + (r0 + j) * s;
-            const uint8_t tf = BSYNC ? (uint8_t)0 : type[c];
+                for (int v = 0; v < 4; v++) put_hint<NT>(ptr_byte(out.f[v], c), t0[v][j] + dd[v][j]);
+            } else {
+                const uint8_t tf = type[(uint32_t)c / (uint32_t)sizeof(T)];
+                const int role = bit_role(nin, j);
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                T x = t0[v][j] + dd[v][j];
-                if (!BSYNC && dirichlet_row(role[j], tf, v < 3 ? 0 : 1)) x = gval[v][c];
-                if (stores & 1) put_hint<NT>(&out.f[v][c], x);
-                if ((stores & 2) && role[j] == RL_IN) put_hint<NT>(&tout.f[v][c], t0[v][j] + km * dd[v][j]);
+                for (int v = 0; v < 4; v++) {
+                    T x = t0[v][j] + dd[v][j];
+                    if (dirichlet_row(role, tf, v < 3 ? 0 : 1)) x = at_byte(gval[v], c);
+                    put_hint<NT>(ptr_byte(out.f[v], c), x);
+                }
+            }
+        };
+        auto put_t = [&](int j) {
+            const int c = rs.first + j * rs.step;
+#pragma unroll
+            for (int v = 0; v < 4; v++) put_hint<NT>(ptr_byte(tout.f[v], c), t0[v][j] + km * dd[v][j]);
+        };
+        if (stores & 1) {
+            if (mixed) {
+#pragma unroll
+                for (int j = 0; j < M; j++)
+                    if ((sys >> (j + 1)) & 1) put_x(j);
+            } else {
+#pragma unroll
+                for (int j = 0; j < M; j++) put_x(j);
+            }
+        }
+        if (stores & 2) {
+            if (mixed) {
+#pragma unroll
+                for (int j = 0; j < M; j++)
+                    if (!((nin >> (j + 1)) & 1)) put_t(j);
+            } else {
+#pragma unroll
+                for (int j = 0; j < M; j++) put_t(j);
             }
         }
     });
+}
+
+template <class T>
+__device__ __forceinline__ Layer4<T> shift_layer(const Layer4<T>& L, int64_t off) {
+    Layer4<T> r;
+#pragma unroll
+    for (int v = 0; v < 4; v++) r.f[v] = L.f[v] + off;
+    return r;
 }
 
 // Row pitch (elements) of the LDS copy of the Picard layer: LPG lines plus
@@ -348,7 +455,6 @@ __device__ __forceinline__ void strided_tile(const InstDesc<T>* __restrict__ ins
     const int gl = lane % LPG;
     const int chunk = wave * GPW + lane / LPG;
     const int P = nw * GPW;
-    const RedLayout L{2 * P, kRedFields * 2 * P + 1};
 
     // work item: the instance and up to kmax of its tiles (tile = outer *
     // ztiles + z tile, -1 = none).  The work-group is sized for the longest
@@ -363,6 +469,7 @@ __device__ __forceinline__ void strided_tile(const InstDesc<T>* __restrict__ ins
     const Geom g = insts[inst].g;
     SweepParams<T> p = insts[inst].p[AXIS];
     p.three_dt = three_dt;
+    const T bv = uniform(three_dt + 2 * p.vis_v), bt = uniform(three_dt + 2 * p.vis_t);
     const int n = AXIS == AX_X ? g.nx : g.ny;
     const int s = AXIS == AX_X ? (int)g.sx : (int)g.sy;
     const int cpl = (n + M - 1) / M;  // chunks per line of this grid
@@ -372,76 +479,41 @@ __device__ __forceinline__ void strided_tile(const InstDesc<T>* __restrict__ ins
     const int outer = tile >= 0 ? tile / ztiles : 0;
     const int z = (tile >= 0 ? tile % ztiles : 0) * LPG + gl;
     const bool zok = tile >= 0 && z < g.nz;
-    // a grid of a batch holds fewer than 2^31 nodes with its offset (checked at
-    // creation): 32-bit element indices
-    const int off = (int)insts[inst].off;
-    const int base = off + (AXIS == AX_X ? outer * (int)g.sy : outer * (int)g.sx) + z;
-    // interior node (1, 1, 1): the element read by rows outside the line
-    const int safe = off + (int)g.sx + (int)g.sy + 1;
+    // the grid's own arrays, and its rows as byte offsets in them (lines of a
+    // tile have x, y in [1, n-2] across the sweep: their neighbour lines exist)
+    const int64_t off = insts[inst].off;
+    const uint8_t* const gt = type + off;
+    const Layer4<T> gin = shift_layer(in, off), gtin = shift_layer(tin, off), gout = shift_layer(out, off),
+                    gtout = shift_layer(tout, off);
+    const T* gg[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) gg[v] = gval[v] + off;
+    const int base = (AXIS == AX_X ? outer * (int)g.sy : outer * (int)g.sx) + z;
+    const int none = (int)g.sx + 1;  // face node (1, 0, 1)
     const int r0 = (chunk - k * cpl) * M;  // first row of the chunk in its line
+    constexpr int B = (int)sizeof(T);
+    const RowSpan rs{(zok ? base : none) * B, (zok ? base + (n - 1) * s : none) * B, (base + r0 * s) * B, s * B};
+    const int sa = (AXIS == AX_X ? (int)g.sy : (int)g.sx) * B;
 
     // KEEP: each lane parks the Picard layer of its rows in LDS, after the
     // reduced systems, [field][row][line], with a padded line pitch (the lane
     // groups of a wave then hit different banks) where the LDS has room for
-    // it; only the lane itself reads it.  The reduced systems then take the
-    // 8-value normalised form (kNormFields), which leaves 128-byte tiles room
-    // for the parked layer.
-    const int red_elems = KEEP ? LPG * kNormFields * pow2_at_least(P) : LPG * L.pitch;
+    // it; only the lane itself reads it.
+    const int red_elems = ends_elems(LPG, P);
     const int krs = keep_row_pitch<T>(LPG, M);
     const int kfs = P * M * krs;
     T* keep = red + red_elems + chunk * M * krs + gl;
-    int role[M];
+    uint32_t nin;
+    bool mixed;
     Chunk<T, M> ch;
     T f[kRedFields], l[kRedFields];
-    strided_chunk<T, AXIS, M, KEEP, BSYNC>(g, p, type, gval, in, tin, base, s, safe, r0, n, zok,
-                                           role, ch, f, l, keep, kfs, krs);
+    strided_chunk<T, AXIS, M, KEEP, BSYNC>(p, bv, bt, gt, gg, gin, gtin, rs, sa, nin, mixed, ch, f,
+                                           l, keep, kfs, krs);
     T xf[4], xl[4];
-    if constexpr (KEEP) {
-        const NormLayout NL{pow2_at_least(P)};
-        T fh[kNormFields];
-        normalise_first<T>(f, fh);
-#pragma unroll
-        for (int k = 0; k < kNormFields; k++) red[NL.at(gl, k, chunk)] = fh[k];
-        __syncthreads();
-        {
-            T nx[kNormFields], cr[kNormFields];
-            const bool hn = chunk + 1 < P;
-#pragma unroll
-            for (int k = 0; k < kNormFields; k++) nx[k] = hn ? red[NL.at(gl, k, chunk + 1)] : (T)0;
-            compact_norm<T>(fh, l, nx, cr);
-            __syncthreads();  // every lane has read the first rows
-#pragma unroll
-            for (int k = 0; k < kNormFields; k++) red[NL.at(gl, k, chunk)] = cr[k];
-        }
-        __syncthreads();
-        solve_norm_lines<T>(red, NL, LPG, P, wave, nw);
-        __syncthreads();
-        if (!zok) return;
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int q = v < 3 ? 0 : 1;
-            xl[v] = red[NL.at(gl, 4 + v, chunk)];
-            const T xlp = chunk > 0 ? red[NL.at(gl, 4 + v, chunk - 1)] : (T)0;
-            xf[v] = fh[4 + v] - fh[2 * q] * xlp - fh[2 * q + 1] * xl[v];
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < kRedFields; k++) {
-            red[L.at(gl, k, 2 * chunk)] = f[k];
-            red[L.at(gl, k, 2 * chunk + 1)] = l[k];
-        }
-        __syncthreads();
-        solve_reduced_compact<T>(red, L, LPG, wave, nw);
-        __syncthreads();
-        if (!zok) return;
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            xf[v] = red[L.at(gl, 6 + v, 2 * chunk)];
-            xl[v] = red[L.at(gl, 6 + v, 2 * chunk + 1)];
-        }
-    }
-    strided_write<T, M, KEEP, BSYNC>(ch, role, type, base, s, safe, r0, xf, xl, gval, tin, out,
-                                     tout, merges, stores, keep, kfs, krs);
+    chunk_ends<T>(red, gl, LPG, chunk, P, wave, nw, f, l, xf, xl);
+    if (!zok) return;
+    strided_write<T, M, KEEP, BSYNC>(ch, nin, mixed, gt, rs, xf, xl, gg, gtin, gout, gtout, merges,
+                                     stores, keep, kfs, krs);
 }
 
 // ---------------------------------------------------------------------------
@@ -500,6 +572,7 @@ __global__ void __launch_bounds__(64 * kZWaves * (LPL / 32), MINW) fused_z_kerne
     const Geom g = insts[inst].g;
     SweepParams<T> p = insts[inst].p[AX_Z];
     p.three_dt = three_dt;
+    const T bv = uniform(three_dt + 2 * p.vis_v), bt = uniform(three_dt + 2 * p.vis_t);
 
     // 2 * kZWaves slots per work-group, 64 / LPL per wavefront.  A slot holds a
     // run of `cnt` consecutive z lines starting at line x*ny + y (-1 = none):
@@ -563,30 +636,23 @@ __global__ void __launch_bounds__(64 * kZWaves * (LPL / 32), MINW) fused_z_kerne
         }
     }
 
-    // node types of the chunk and of the rows either side (from the neighbour lanes)
-    uint8_t ty[M + 2];
+    // row bits of the chunk and of the rows either side (from the neighbour
+    // lanes; a slot starts and ends on a face node), see bit_role
+    uint32_t nin = 0, any = 0;
 #pragma unroll
-    for (int j = 0; j < M; j++) ty[j + 1] = j < valid ? (uint8_t)tyr[j] : kOutside;
+    for (int j = 0; j < M; j++) {
+        nin |= (j < valid ? min((uint32_t)tyr[j], 1u) : 1u) << (j + 1);
+        any |= j < valid ? (uint32_t)tyr[j] : 0u;
+    }
     {
-        int prev = lane_prev((int)ty[M]);
-        int next = lane_next((int)ty[1]);
-        ty[0] = (ll > 0 && ok) ? (uint8_t)prev : kOutside;
-        ty[M + 1] = (ll < LPL - 1 && ok && r0 + M < n) ? (uint8_t)next : kOutside;
+        const uint32_t prev = ((uint32_t)lane_prev((int)nin) >> M) & 1u;
+        const uint32_t next = ((uint32_t)lane_next((int)nin) >> 1) & 1u;
+        nin |= (ll > 0 ? prev : 1u) | (ll < LPL - 1 ? next : 1u) << (M + 1);
     }
-    int role[M];
-#pragma unroll
-    for (int j = 0; j < M; j++) role[j] = row_role(ty[j + 1], ty[j], ty[j + 2]);
-    // Dirichlet values of the boundary rows (ApplyBC0/1; the BC kinds are in
-    // the flags bytes): the Picard layer while the state is in sync with the
-    // node values (it holds them off NODE_IN), else the node values of the
-    // whole chunk, loaded above (a load per boundary row would sit inside the
-    // elimination chain)
-    if (bsync) {
-#pragma unroll
-        for (int j = 0; j < M; j++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) gb[v][j] = 0;
-    }
+    // rows with a value of their own (ApplyBC0/1): free ends, and every boundary
+    // row while the state is out of sync with the node values; the Picard layer
+    // holds the others' values
+    const bool special = !bsync || __any((any & (kFlagFreeVel | kFlagFreeT)) != 0);
     T wx[M], wy[M];
 #pragma unroll
     for (int j = 0; j < M; j++) {
@@ -621,23 +687,27 @@ __global__ void __launch_bounds__(64 * kZWaves * (LPL / 32), MINW) fused_z_kerne
 #pragma unroll
     for (int j = 0; j < M; j++) {
         // correction form (see interior_row_delta): Picard layer around the row
-        T wm[4], w0[4], wp[4], ci[4], gd[4];
+        T wm[4], w0[4], wp[4], ci[4];
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             wm[v] = j > 0 ? tv[v][j - 1] : tprev[v];
             w0[v] = tv[v][j];
             wp[v] = j < M - 1 ? tv[v][j + 1] : tnext[v];
             ci[v] = cu[v][j];
-            gd[v] = bsync ? w0[v] : gb[v][j];
         }
-        Row<T> ri, rb, r;
-        interior_row_delta<T, AX_Z>(p, wm, w0, wp, ci, wx[j], wy[j], ri);
-        boundary_row_delta<T>(role[j], ty[j + 1], wm, w0, wp, gd, rb);
-        const bool isin = role[j] == RL_IN;
-        r.av = isin ? ri.av : rb.av; r.bv = isin ? ri.bv : rb.bv; r.cv = isin ? ri.cv : rb.cv;
-        r.at = isin ? ri.at : rb.at; r.bt = isin ? ri.bt : rb.bt; r.ct = isin ? ri.ct : rb.ct;
+        Row<T> r;
+        interior_row_delta<T, AX_Z>(p, bv, bt, wm, w0, wp, ci, wx[j], wy[j], r);
+        const bool isin = !((nin >> (j + 1)) & 1);
+        if (!special) {
+            keep_or_identity<T>(isin, r);
+        } else {
+            T gd[4];
 #pragma unroll
-        for (int v = 0; v < 4; v++) r.d[v] = isin ? ri.d[v] : rb.d[v];
+            for (int v = 0; v < 4; v++) gd[v] = bsync ? w0[v] : gb[v][j];
+            Row<T> rb;
+            boundary_row_delta<T>(bit_role(nin, j), (uint8_t)tyr[j], wm, w0, wp, gd, rb);
+            if (!isin) r = rb;
+        }
         if (j == 0) rfirst = r;
         else if (j == M - 1) rlast = r;
         else chunk_down<T, M>(ch, j, r);
@@ -667,31 +737,43 @@ __global__ void __launch_bounds__(64 * kZWaves * (LPL / 32), MINW) fused_z_kerne
             }
     }
     const T km = merges > 1 ? (T)0.75 : (T)0.5;
+    const uint32_t sys = system_rows(nin);
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+#pragma unroll
+        for (int j = 0; j < M; j++) {
+            T d;  // correction of row j (xf / xl: of the chunk's first / last row)
+            if (j == 0) d = xf[v];
+            else if (j == M - 1) d = xl[v];
+            else {
+                const T F = v < 3 ? ch.Fv[j] : ch.Ft[j];
+                const T G = v < 3 ? ch.Gv[j] : ch.Gt[j];
+                d = ch.E[v][j] + F * xf[v] + G * xl[v];
+            }
+            // rows no segment covers keep the sweep input's value; x in cu, the
+            // merged layer in tv (d is zero on other rows than NODE_IN ones
+            // unless they have a value of their own)
+            T x = tv[v][j] + d;
+            if (special) {
+                if (!bsync && dirichlet_row(bit_role(nin, j), (uint8_t)tyr[j], v < 3 ? 0 : 1)) x = gb[v][j];
+                if ((nin >> (j + 1)) & 1) d = 0;
+            }
+            cu[v][j] = (sys >> (j + 1)) & 1 ? x : cu[v][j];
+            tv[v][j] = tv[v][j] + km * d;
+        }
+    }
     with_store_hint((stores & kStoreStream) != 0, [&](auto ntc) {
         constexpr bool NT = decltype(ntc)::value;
+        auto put = [&](bool all) {
+            if (stores & 1)
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-            T x[M], t[M];
+                for (int v = 0; v < 4; v++) store_run<T, M, NT>(out.f[v] + c0, cu[v], all, valid);
+            if (stores & 2)
 #pragma unroll
-            for (int j = 0; j < M; j++) {
-                T d;  // correction of row j (xf / xl: of the chunk's first / last row)
-                if (j == 0) d = xf[v];
-                else if (j == M - 1) d = xl[v];
-                else {
-                    const T F = v < 3 ? ch.Fv[j] : ch.Ft[j];
-                    const T G = v < 3 ? ch.Gv[j] : ch.Gt[j];
-                    d = ch.E[v][j] + F * xf[v] + G * xl[v];
-                }
-                x[j] = tv[v][j] + d;
-                if (!bsync && dirichlet_row(role[j], ty[j + 1], v < 3 ? 0 : 1)) x[j] = gb[v][j];
-                // rows no segment covers get the sweep input's value
-                if (role[j] == RL_NONE) x[j] = cu[v][j];
-                t[j] = role[j] == RL_IN ? tv[v][j] + km * d : tv[v][j];
-            }
-            // whole runs: partial-vector stores would cost far more than the bytes
-            if (stores & 1) store_run<T, M, NT>(out.f[v] + c0, x, whole, valid);
-            if (stores & 2) store_run<T, M, NT>(tout.f[v] + c0, t, whole, valid);
-        }
+                for (int v = 0; v < 4; v++) store_run<T, M, NT>(tout.f[v] + c0, tv[v], all, valid);
+        };
+        if (whole) put(true);
+        else put(false);
     });
 }
 
@@ -747,9 +829,8 @@ template <class T>
 size_t strided_lds(int n, int v) {
     const int lpg = variant_lpg<T>(v), m = variant_chunk<T>(v);
     const int P = strided_waves_for(n, lpg, m) * (64 / lpg);
-    if (!kShapes[v].keep) return (size_t)lpg * (kRedFields * 2 * P + 1) * sizeof(T);
-    return (size_t)lpg * kNormFields * pow2_at_least(P) * sizeof(T) +
-           (size_t)4 * P * m * keep_row_pitch<T>(lpg, m) * sizeof(T);
+    return (size_t)ends_elems(lpg, P) * sizeof(T) +
+           (kShapes[v].keep ? (size_t)4 * P * m * keep_row_pitch<T>(lpg, m) * sizeof(T) : 0);
 }
 
 // A strided variant fits lines of n nodes when its work-group (one lane per

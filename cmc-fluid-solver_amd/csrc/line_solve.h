@@ -161,9 +161,30 @@ __device__ __forceinline__ double lane_next(double x) {
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
+// Off-diagonals (of a row divided by its diagonal) that no longer count: the
+// neighbours' part of x is then below 2^-24 of the rounding of a neighbour's
+// own x (FP32; FP64 below 2^-43 of it).  Every reduction step about squares the
+// off-diagonals, and eliminating a chunk of M rows already raises a row's
+// off-diagonal ratio to about its M-th power: with dt |w| / 6 h + dt nu / 3 h^2
+// = 0.01 to 0.1, the range of the configured flows, the rows of 8-row chunks
+// are decoupled after 0 to 2 of the 5 steps that 32 chunks would take.  A row
+// with an infinite or NaN right-hand side counts as coupled, so that such a
+// value spreads over its line as a full solve spreads it.
+template <class T>
+__device__ __forceinline__ bool decoupled(const T* A, const T* C, const T* D) {
+    constexpr T tiny = sizeof(T) == 4 ? (T)0x1p-48 : (T)0x1p-96;
+    bool ok = true;
+#pragma unroll
+    for (int q = 0; q < 2; q++) ok = ok && fabs(A[q]) <= tiny && fabs(C[q]) <= tiny;
+#pragma unroll
+    for (int v = 0; v < 4; v++) ok = ok && __builtin_isfinite(D[v]);
+    return ok;
+}
+
 // Parallel cyclic reduction over one reduced system per group of RP lanes:
 // the lane holds row i = lane % RP (rows >= R are identity, and every access
-// stays inside the lane's group).  On return D holds x.
+// stays inside the lane's group), until the rows of the whole wavefront are
+// decoupled.  On return D holds x.
 template <class T>
 __device__ __forceinline__ void pcr_solve(T* A, T* B, T* C, T* D, int i, int R, int RP) {
     // A[q], B[q], C[q]: matrix q (0 vel, 1 T); D[0..2] use matrix 0, D[3] matrix 1.
@@ -186,6 +207,7 @@ __device__ __forceinline__ void pcr_solve(T* A, T* B, T* C, T* D, int i, int R, 
     }
     const int lane = threadIdx.x & 63;
     for (int st = 1; st < RP; st <<= 1) {
+        if (__all(decoupled<T>(A, C, D))) break;
         const bool hm = i - st >= 0, hp = i + st < RP;
         const int lm = hm ? lane - st : lane, lp = hp ? lane + st : lane;
         T Am[2], Cm[2], Ap[2], Cp[2], Dm[4], Dp[4];
@@ -230,13 +252,6 @@ __device__ __forceinline__ void pcr_solve(T* A, T* B, T* C, T* D, int i, int R, 
             C[q] = c * ib;
         }
     }
-}
-
-// Identity reduced row (x = 0) in the kRedFields layout.
-template <class T>
-__device__ __forceinline__ void ident_row(T* r) {
-#pragma unroll
-    for (int k = 0; k < kRedFields; k++) r[k] = (k == 1 || k == 4) ? (T)1 : (T)0;
 }
 
 // One cyclic-reduction step on the reduced system (2 rows per chunk): chunk i's
@@ -303,73 +318,14 @@ __device__ __forceinline__ void solve_chunks_in_lanes(const T* f, const T* l, in
     first_unknowns<T>(f, ib, xlp, xl, xf);
 }
 
-// Reduced systems staged in LDS as [line][field][row] with a line pitch of
-// kRedFields*R + 1 elements (conflict-free for both the chunk writes, one lane
-// per line, and the PCR reads, one lane per row).
-struct RedLayout {
-    int R, pitch;
-    __device__ __forceinline__ int at(int line, int field, int row) const {
-        return line * pitch + field * R + row;
-    }
-};
-
-// Solves `nl` reduced systems held in LDS (row 2i = f_i, row 2i+1 = l_i of
-// chunk i, L.R / 2 chunks per line) with the lanes of `nw` wavefronts (this one
-// is wave `w`): compaction to one unknown per chunk, one lane per chunk with the
-// lanes of a line inside one wavefront, PCR over L.R / 2 rows; writes x_f and
-// x_l over the D fields of rows 2i and 2i+1.
-template <class T>
-__device__ __forceinline__ void solve_reduced_compact(T* red, RedLayout L, int nl, int w, int nw) {
-    const int lane = threadIdx.x & 63;
-    const int P = L.R / 2;
-    int RP = 1;
-    while (RP < P) RP <<= 1;
-    const int lpp = 64 / RP;  // lines per pass of one wave
-    const int i = lane % RP;
-    for (int base = w * lpp; base < nl; base += nw * lpp) {
-        const int line = base + lane / RP;
-        const int Rl = line < nl ? P : 0;
-        const bool act = i < Rl, actn = i + 1 < Rl;
-        T f[kRedFields], l[kRedFields], fn[kRedFields];
-#pragma unroll
-        for (int k = 0; k < kRedFields; k++) {
-            const T id = (k == 1 || k == 4) ? (T)1 : (T)0;
-            f[k] = act ? red[L.at(line, k, 2 * i)] : id;
-            l[k] = act ? red[L.at(line, k, 2 * i + 1)] : id;
-            fn[k] = actn ? red[L.at(line, k, 2 * i + 2)] : id;
-        }
-        T A[2], B[2], C[2], D[4], ib[2];
-        compact_rows<T>(f, l, fn, A, B, C, D, ib);
-        pcr_solve<T>(A, B, C, D, i, Rl, RP);
-        T xlp[4], xl[4], xf[4];
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const T t = lane_prev(D[v]);
-            xlp[v] = i > 0 ? t : (T)0;
-            xl[v] = D[v];
-        }
-        first_unknowns<T>(f, ib, xlp, xl, xf);
-        // the reads of row 2i+2 above (lane i) precede this write (lane i+1,
-        // same wavefront) in program order
-        if (act) {
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                red[L.at(line, 6 + v, 2 * i)] = xf[v];
-                red[L.at(line, 6 + v, 2 * i + 1)] = xl[v];
-            }
-        }
-    }
-}
-
-// Reduced system in 8 values per chunk, for kernels whose LDS is mostly taken
-// by other data: the chunk's lane divides its first row by b and stores it;
-// after a barrier it reads the next chunk's normalised first row, eliminates
-// both first unknowns from its last row (the compaction step above) and stores
-// that row, again divided by its b.  PCR then runs over one row per chunk, and
-// each lane recovers x_f from its own normalised first row.  Row i of line
-// `line` is at NormLayout::at; chunks are XOR-swizzled by the line so that the
-// chunk-major stores (lanes = lines) and the line-major PCR loads (lanes =
-// chunks) both spread over the banks.
+// Reduced systems of lines whose chunks span wavefronts, in LDS.  A chunk's lane
+// divides its first row by b and stores it (8 values); after a barrier it reads
+// the next chunk's normalised first row and eliminates both first unknowns from
+// its last row (the compaction step above).  PCR over these rows, one per chunk,
+// gives the last unknowns, and each lane recovers x_f from its own first row.
+// Row i of line `line` is at NormLayout::at; chunks are XOR-swizzled by the line
+// so that the chunk-major stores (lanes = lines) and the line-major PCR loads
+// (lanes = chunks) both spread over the banks.
 constexpr int kNormFields = 8;  // a_v c_v a_t c_t d_u d_v d_w d_t, over the row's b
 struct NormLayout {
     int P2;  // chunks per line rounded up to a power of two
@@ -397,19 +353,25 @@ __device__ __forceinline__ void normalise_first(const T* f, T* fh) {
     }
 }
 
-// Last row l with this chunk's (fh) and the next chunk's (nx, zeros past the
-// line's end) normalised first rows substituted; normalised result in cr.
-template <class T>
-__device__ __forceinline__ void compact_norm(const T* fh, const T* l, const T* nx, T* cr) {
+// Last row l with this chunk's (fh) and the next chunk's normalised first rows
+// substituted; normalised result in cr.  next(k): field k of the next chunk's
+// row (zero past the line's end), read one matrix at a time to spare registers.
+template <class T, class F>
+__device__ __forceinline__ void compact_norm(const T* fh, const T* l, F next, T* cr) {
 #pragma unroll
     for (int q = 0; q < 2; q++) {
         const T al = l[3 * q], bl = l[3 * q + 1], cl = l[3 * q + 2];
-        const T iB = rcp(bl - al * fh[2 * q + 1] - cl * nx[2 * q]);
+        const T na = next(2 * q), nc = next(2 * q + 1);
+        T nd[3];
+#pragma unroll
+        for (int v = (q == 0 ? 0 : 3); v < (q == 0 ? 3 : 4); v++) nd[v - 3 * q] = next(4 + v);
+        const T iB = rcp(bl - al * fh[2 * q + 1] - cl * na);
         cr[2 * q] = -al * fh[2 * q] * iB;
-        cr[2 * q + 1] = -cl * nx[2 * q + 1] * iB;
+        cr[2 * q + 1] = -cl * nc * iB;
 #pragma unroll
         for (int v = (q == 0 ? 0 : 3); v < (q == 0 ? 3 : 4); v++)
-            cr[4 + v] = (l[6 + v] - al * fh[4 + v] - cl * nx[4 + v]) * iB;
+            cr[4 + v] = (l[6 + v] - al * fh[4 + v] - cl * nd[v - 3 * q]) * iB;
+        __builtin_amdgcn_sched_barrier(0);
     }
 }
 
@@ -439,6 +401,60 @@ __device__ __forceinline__ void solve_norm_lines(T* red, NormLayout NL, int nl, 
 #pragma unroll
             for (int v = 0; v < 4; v++) red[NL.at(line, 4 + v, i)] = D[v];
         }
+    }
+}
+
+// LDS elements of chunk_ends for nl lines of P chunks.
+__host__ __device__ constexpr int ends_elems(int nl, int P) { return nl * kNormFields * pow2_at_least(P); }
+
+// First and last unknowns of the lane's chunk (line gl of nl, chunk of P <= 64)
+// from its reduced rows f, l.  Where every row of the work-group is decoupled
+// after the compaction, its right-hand side is the last unknown, and only the
+// previous chunk's is still exchanged: 24 LDS accesses per lane and no PCR,
+// whose lanes would wait on one another's permutes.  Each wavefront votes in a
+// word that nothing else uses then (field 0 of line `wave`, chunk 0: no chunk
+// reads chunk 0's first row).  Every thread of the work-group must call it.
+template <class T>
+__device__ __forceinline__ void chunk_ends(T* red, int gl, int nl, int chunk, int P, int wave, int nw,
+                                           const T* f, const T* l, T* xf, T* xl) {
+    const NormLayout NL{pow2_at_least(P)};
+    T fh[kNormFields], cr[kNormFields];
+    normalise_first<T>(f, fh);
+    if (chunk > 0) {
+#pragma unroll
+        for (int k = 0; k < kNormFields; k++) red[NL.at(gl, k, chunk)] = fh[k];
+    }
+    __syncthreads();
+    const bool hn = chunk + 1 < P;
+    compact_norm<T>(fh, l, [&](int k) { return hn ? red[NL.at(gl, k, chunk + 1)] : (T)0; }, cr);
+    {
+        const T A[2] = {cr[0], cr[2]}, C[2] = {cr[1], cr[3]};
+        const bool dec = __all(decoupled<T>(A, C, cr + 4));
+        if ((threadIdx.x & 63) == 0) red[NL.at(wave, 0, 0)] = dec ? (T)1 : (T)0;
+    }
+    __syncthreads();  // the votes are in, and every lane has read the first rows
+    const int lane = threadIdx.x & 63;
+    if (__all(red[NL.at(lane < nw ? lane : 0, 0, 0)] != (T)0)) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) red[NL.at(gl, 4 + v, chunk)] = cr[4 + v];
+        __syncthreads();
+#pragma unroll
+        for (int v = 0; v < 4; v++) xl[v] = cr[4 + v];
+    } else {
+        __syncthreads();  // the votes have been read
+#pragma unroll
+        for (int k = 0; k < kNormFields; k++) red[NL.at(gl, k, chunk)] = cr[k];
+        __syncthreads();
+        solve_norm_lines<T>(red, NL, nl, P, wave, nw);
+        __syncthreads();
+#pragma unroll
+        for (int v = 0; v < 4; v++) xl[v] = red[NL.at(gl, 4 + v, chunk)];
+    }
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int q = v < 3 ? 0 : 1;
+        const T xp = chunk > 0 ? red[NL.at(gl, 4 + v, chunk - 1)] : (T)0;
+        xf[v] = fh[4 + v] - fh[2 * q] * xp - fh[2 * q + 1] * xl[v];
     }
 }
 
