@@ -802,6 +802,351 @@ __global__ void __launch_bounds__(1024) k2s_poisson(
     }
 }
 
+// The relaxation for grids whose q fits the LDS, the form that the solver
+// picks whenever it does (the two fronts, the lag of kPoisLag steps between
+// sweeps and the stopping test are those of k2s_poisson above, and so is every
+// value).  Both run on one compute unit and are bound by the instructions that
+// its wavefronts issue; k2s_poisson makes 10 reads, 6 clamped addresses and both
+// fronts' arithmetic for every lane and step, half of its lanes outside the
+// front (284 steps of 2700 cycles for 8 sweeps of a 120 x 135 grid).  Here:
+//   * q lies in LDS by anti-diagonals: cell (r, j), x = j + 1, is element
+//     ((x + r) mod P, r + 1) of P rows of nx + 2.  A front is one row, a lane's
+//     neighbours are in the rows either side, and the lanes' accesses are
+//     consecutive.  x = 0 and the first and last elements of a row hold zero;
+//     P >= ny + 1, so that x = 0 also ends a grid row.
+//   * slices of rp threads (rp >= nx) relax inner cells, lane r row r, for MW
+//     sweeps each (D in all), one cell of each per step, and start their next
+//     sweeps P steps after the last ones' start without waiting for the other
+//     rows: no lane idles at the ends of a front.  Sweep n starts at step
+//     (n mod D) kPoisLag + (n div D) P, at least kPoisLag after sweep n - 1
+//     (P >= kPoisLag D), which is all that the order needs.  At residue
+//     (x + r) mod P the rows r <= residue of a wavefront are in its newest
+//     sweep, the others still in the one before: P >= nx, or P is a multiple
+//     of 64 and each wavefront has its own delay.
+//   * a cell's own value comes from the last step's right neighbour, its left
+//     one from the last step's result.
+//   * the few boundary cells of a front are relaxed for all D sweeps by bw
+//     wavefronts of their own, from lists per residue.
+//   * an inner cell's div dx2 dy2 comes from `dvs`, laid out like q, two steps
+//     ahead; kNotInner marks the other cells, so that no flags are read.
+//   * the stopping test works on lane masks, in scalar registers: per sweep and
+//     row a NaN, and a change of tol or more since the row's last NaN.
+// Per sweep of a 120 x 135 grid in FP64: 39.6 us before, 7.0 now; with one sweep
+// per lane 8.2, with four 8.6 (scalar registers spill).  A first form with rows
+// of q in LDS, where a lane moves on to its next sweep by itself in a branch
+// that some lane takes on every step, took 7.7 to 8.6.
+constexpr int kPoisGroup = 256;              // sweeps of a group at most
+constexpr unsigned kNotInner = 0x7ff5a5a5u;  // high word of dvs off the inner cells (no result is this NaN)
+constexpr int kDvRows = kPoisLag;            // rows of dvs repeated before the first
+constexpr uint32_t kBValid = 1u << 28;
+// Boundary list entry: x: place in sweep order (r P + x), selects << 16, kBValid;
+// y: r, (x + r) / P << 16.
+
+// Whether |(qn - qo) / qn| >= tol: the sign of |qn - qo| - tol |qn| away from
+// zero (`eps` = tol times a margin far above the rounding of either side; the
+// tiny constant keeps the margin where tol |qn| underflows): yes if t > b, no if
+// t < -b, otherwise (infinite or NaN values too) change_divided decides.
+__device__ __forceinline__ void change_sides(double qn, double qo, double tol, double eps, double& t, double& b) {
+    const double m = fabs(qn);
+    t = __builtin_fma(m, -tol, fabs(qn - qo));
+    b = __builtin_fma(m, eps, 1e-300);
+}
+__device__ __forceinline__ bool change_divided(double qn, double qo, double tol, bool& nan) {
+    const double ce = fabs((qn - qo) / qn);
+    nan = ce != ce;
+    return ce >= tol;
+}
+
+template <class T, int MW>
+__global__ void __launch_bounds__(1024) k2s_poisson_lds(
+    int nx, int P, int rp, int D, int bw, int cpad, const uint2* __restrict__ blist,
+    const double* __restrict__ dvs, T* __restrict__ qgrid, T* __restrict__ save, double dx2,
+    double dy2, double rcp, double tol, int max_sweeps, int resume, int32_t* __restrict__ status) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    // per sweep: the last place in sweep order with a change >= tol, with a NaN
+    // (0 = none)
+    __shared__ int fold[2 * kPoisGroup];
+    __shared__ int s_first;
+    __shared__ T dump[64];  // stores of cells that are not inner ones
+    using Lds = __attribute__((address_space(3))) T;
+    using LdsByte = __attribute__((address_space(3))) char;
+    T* const q = reinterpret_cast<T*>(smem);
+    const int Q = nx + 2, S = P * Q;
+    for (int c = threadIdx.x; c < S; c += blockDim.x) q[c] = resume ? qgrid[c] : (T)0;
+    const double eps = tol * 2e-12;
+    auto step_barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    const int nin = D / MW * rp;                // threads of the inner slices
+    const bool inner = (int)threadIdx.x < nin;  // uniform per wave
+    // inner: row r of members mem .. mem + MW - 1; boundary: slot e0 of member mem
+    const int epm = 64 * bw / D;
+    const int lb = (int)threadIdx.x - nin;
+    const int mem = inner ? (int)threadIdx.x / rp * MW : lb / epm;
+    const int r = (int)threadIdx.x - mem / MW * rp, e0 = lb % epm;
+    const int k0 = kPoisLag * mem;
+    auto next = [&](int a) { return a + 1 == P ? 0 : a + 1; };
+
+    int sweeps = resume ? status[0] : 0, left = max_sweeps, rerun = 0, gsize = resume ? kPoisGroup : 16;
+    bool converged = false;
+    __syncthreads();
+    while (left > 0) {
+        const int g = rerun ? rerun : min(gsize, left);  // sweeps of this group (uniform)
+        if (!rerun && g > 1)
+            for (int c = threadIdx.x; c < S; c += blockDim.x) save[c] = q[c];
+        for (int c = threadIdx.x; c < 2 * kPoisGroup; c += blockDim.x) fold[c] = 0;
+        if (threadIdx.x == 0) s_first = g;
+        __syncthreads();
+        // to the end of sweep g - 1: its start, rows, columns and the inner
+        // front's two steps, in whole turns of the loops' four steps
+        const int steps = (((g - 1) / D) * P + ((g - 1) % D) * kPoisLag + nx + P + 2 + 3) & ~3;
+        if (inner) {
+            // Branch-free but for the rare cases (a change too close to tol to
+            // tell, the end of a turn), each tested once for the MW cells.
+            const int w0 = __builtin_amdgcn_readfirstlane(r);  // the wavefront's first row
+            const int late = w0 / P, wr = w0 - late * P;       // its delay in turns, its first row's residue at x = 0
+            const uint64_t rows = nx - w0 >= 64 ? ~0ull : nx > w0 ? (1ull << (nx - w0)) - 1 : 0;
+            const uint32_t qb = (uint32_t)Q * (uint32_t)sizeof(T), pb = (uint32_t)P * qb;  // bytes of a row, of q
+            // lanes beyond the rows read the last one's cells and are never live
+            Lds* const ql = (Lds*)(q + min(r, nx - 1));
+            Lds* const pdump = (Lds*)&dump[threadIdx.x & 63];
+            auto at = [&](uint32_t row) { return (Lds*)((LdsByte*)ql + row); };
+            uint32_t voff[MW], rb[MW], rs[MW], rf[MW];  // rows of residues res - 1, res, res + 1
+            int res[MW], n[MW];                         // per member: residue, newest sweep
+            // lanes in the newest sweep; of these and of the others, those whose
+            // sweep is one of the group's; rows with a change >= tol, with a NaN
+            // in the newest sweep and in the one before
+            uint64_t newest[MW], live1[MW], live0[MW], ge1[MW], ge0[MW], na1[MW], na0[MW];
+            double lft[MW], cur[MW], dv[MW][2];
+            auto set_live = [&](int u) {
+                live1[u] = n[u] >= 0 && n[u] < g ? rows : 0;
+                live0[u] = n[u] >= D && n[u] < g + D ? rows : 0;
+            };
+            // dvs two steps on, its row's residue the first member's
+            const uint32_t db = (uint32_t)rp * (uint32_t)sizeof(double);
+            int res2 = __builtin_amdgcn_readfirstlane((P - (k0 + 2) % P) % P);
+            const char* drow = reinterpret_cast<const char*>(dvs) + (int64_t)res2 * db;
+            auto advance_dvs = [&] {
+                res2++;
+                drow += db;
+                if (res2 == P) {
+                    res2 = 0;
+                    drow = reinterpret_cast<const char*>(dvs);
+                }
+            };
+#pragma unroll
+            for (int u = 0; u < MW; u++) {
+                const int back = __builtin_amdgcn_readfirstlane(k0 + kPoisLag * u + 2), turns = (back + P - 1) / P;
+                res[u] = turns * P - back;
+                n[u] = __builtin_amdgcn_readfirstlane(mem + u - D * (turns + late));
+                const int k1 = res[u] - wr;
+                newest[u] = k1 >= 63 ? ~0ull : k1 >= 0 ? (2ull << k1) - 1 : 0;
+                set_live(u);
+                rs[u] = (uint32_t)res[u] * qb;
+                rb[u] = rs[u] == 0 ? pb - qb : rs[u] - qb;
+                rf[u] = rs[u] + qb == pb ? 0 : rs[u] + qb;
+                voff[u] = (uint32_t)(kDvRows - kPoisLag * u) * db + (uint32_t)r * (uint32_t)sizeof(double);
+                lft[u] = cur[u] = 0;
+                ge1[u] = ge0[u] = na1[u] = na0[u] = 0;
+            }
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+#pragma unroll
+                for (int u = 0; u < MW; u++) dv[u][h] = *reinterpret_cast<const double*>(drow + voff[u]);
+                advance_dvs();
+            }
+            // (waited for here: loads outstanding at the loop's entry would make
+            // every turn wait for its newest ones)
+#pragma unroll
+            for (int u = 0; u < MW; u++) asm volatile("" : "+v"(dv[u][0]), "+v"(dv[u][1]));
+            // a finished sweep's last row with a change >= tol since its last NaN,
+            // and its last NaN; inner cells follow the boundary cells in sweep order
+            auto flush = [&](int m, uint64_t ge, uint64_t na) {
+                if (m < 0 || m >= g || (threadIdx.x & 63) != 0) return;
+                if (ge) atomicMax(&fold[2 * m], 0x10001 + 2 * (w0 + 63 - __builtin_clzll(ge)));
+                if (na) atomicMax(&fold[2 * m + 1], 0x10000 + 2 * (w0 + 63 - __builtin_clzll(na)));
+            };
+            for (int k = 0; k < steps; k += 2) {
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    double rgt[MW], qn[MW], qo[MW];
+                    uint64_t doubt[MW], any = 0;
+#pragma unroll
+                    for (int u = 0; u < MW; u++) {
+                        Lds* const f = at(rf[u]);
+                        const double up = (double)at(rb[u])[0], dn = (double)f[2];
+                        rgt[u] = (double)f[1];
+                        qn[u] = up + dn;
+                    }
+#pragma unroll
+                    for (int u = 0; u < MW; u++) {
+                        const double v = dv[u][h];
+                        int mark = __double2hiint(v);
+                        asm("" : "+v"(mark));
+                        const uint64_t inm = __ballot((unsigned)mark != kNotInner) &
+                                             ((newest[u] & live1[u]) | (~newest[u] & live0[u]));
+                        const bool in = __builtin_amdgcn_inverse_ballot_w64(inm);
+                        qn[u] = rcp * (qn[u] * dy2 + (lft[u] + rgt[u]) * dx2 - v);
+                        qo[u] = cur[u];
+                        *(in ? at(rs[u]) + 1 : pdump) = (T)qn[u];
+                        lft[u] = in ? (double)(T)qn[u] : qo[u];
+                        cur[u] = rgt[u];
+                        double t, b;
+                        change_sides(qn[u], qo[u], tol, eps, t, b);
+                        const uint64_t ge = __ballot(t > b) & inm;
+                        doubt[u] = inm & ~__ballot(fabs(t) > b);
+                        any |= doubt[u];
+                        ge1[u] |= ge & newest[u];
+                        ge0[u] |= ge & ~newest[u];
+                    }
+                    if (any) {
+#pragma unroll
+                        for (int u = 0; u < MW; u++) {
+                            bool nan;
+                            const uint64_t ge = __ballot(change_divided(qn[u], qo[u], tol, nan)) & doubt[u];
+                            const uint64_t na = __ballot(nan) & doubt[u];
+                            ge1[u] = (ge1[u] & ~(na & newest[u])) | (ge & newest[u]);
+                            ge0[u] = (ge0[u] & ~(na & ~newest[u])) | (ge & ~newest[u]);
+                            na1[u] |= na & newest[u];
+                            na0[u] |= na & ~newest[u];
+                        }
+                    }
+#pragma unroll
+                    for (int u = 0; u < MW; u++) {
+                        rb[u] = rs[u];
+                        rs[u] = rf[u];
+                        rf[u] = rf[u] + qb == pb ? 0 : rf[u] + qb;
+                        res[u]++;
+                        if (res[u] == P) {  // a new turn: every row is out of the last sweep
+                            flush(n[u] - D, ge0[u], na0[u]);
+                            ge0[u] = ge1[u];
+                            na0[u] = na1[u];
+                            ge1[u] = na1[u] = 0;
+                            n[u] += D;
+                            set_live(u);
+                            res[u] = 0;
+                            newest[u] = 0;
+                        }
+                        newest[u] = newest[u] << 1 | (uint64_t)(res[u] >= wr);
+                        dv[u][h] = *reinterpret_cast<const double*>(drow + voff[u]);
+                    }
+                    advance_dvs();
+                    step_barrier();
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < MW; u++) {
+                flush(n[u] - D, ge0[u], na0[u]);
+                flush(n[u], ge1[u], na1[u]);
+            }
+        } else {
+            __builtin_amdgcn_s_setprio(3);  // the longest chain of a step
+            const bool mine = mem < D;
+            // step - k0 = turn P + res (lanes beyond the last member's: any diagonal)
+            int res = mine && k0 ? P - k0 : 0, turn = mine && k0 ? -1 : 0;
+            const uint2* const bl = blist + (mine ? e0 : 0);
+            uint2 w[4];
+            int pre = res;
+#pragma unroll
+            for (int h = 0; h < 4; h++) {
+                w[h] = bl[pre * cpad];
+                pre = next(pre);
+            }
+            // relaxes the cell of a list entry, if its sweep is one of the group's
+            auto relax = [&](uint2 e) {
+                const int n = (turn - (int)(e.y >> 16)) * D + mem;
+                if (!mine || !(e.x & kBValid) || n < 0 || n >= g) return;
+                T* const c = q + (e.y & 0xffff);
+                T* const b = c + (res == 0 ? P - 1 : res - 1) * Q;
+                T* const s = c + res * Q + 1;
+                const T* const f = c + next(res) * Q;
+                const double qo = (double)s[0], lf = (double)b[1], rt = (double)f[1];
+                const double up = (double)b[0], dn = (double)f[2];
+                const double i0 = e.x & (1u << 16) ? up : dn, i1 = e.x & (1u << 17) ? dn : up;
+                const double j0 = e.x & (1u << 18) ? lf : rt, j1 = e.x & (1u << 19) ? rt : lf;
+                // div is zero on boundary cells
+                const double qn = rcp * ((i0 + i1) * dy2 + (j0 + j1) * dx2 - 0.0);
+                s[0] = (T)qn;
+                double t, m;
+                change_sides(qn, qo, tol, eps, t, m);
+                bool nan = false, ge = t > m;
+                if (!(fabs(t) > m)) ge = change_divided(qn, qo, tol, nan);
+                if (ge) atomicMax(&fold[2 * n], (int)(e.x & 0xffff));
+                if (nan) atomicMax(&fold[2 * n + 1], (int)(e.x & 0xffff));
+            };
+            for (int k = 0; k < steps; k += 4) {
+#pragma unroll
+                for (int h = 0; h < 4; h++) {
+                    relax(w[h]);
+                    w[h] = bl[pre * cpad];  // after its use: no wait for this load before the next step's
+                    pre = next(pre);
+                    for (int e = epm; e < cpad; e += epm) relax(bl[res * cpad + e]);
+                    res = next(res);
+                    if (res == 0) turn++;
+                    step_barrier();
+                }
+            }
+            __builtin_amdgcn_s_setprio(0);
+        }
+        __syncthreads();
+        for (int n = threadIdx.x; n < g; n += blockDim.x)
+            if (fold[2 * n] <= fold[2 * n + 1]) atomicMin(&s_first, n);
+        __syncthreads();
+        const int first = s_first;
+        if (rerun || first + 1 == g) {  // a rerun ends on its last sweep
+            sweeps += g;
+            converged = true;
+            break;
+        }
+        if (first < g) {
+            for (int c = threadIdx.x; c < S; c += blockDim.x) q[c] = save[c];
+            rerun = first + 1;
+            __syncthreads();
+            continue;
+        }
+        sweeps += g;
+        left -= g;
+        gsize = min(2 * gsize, kPoisGroup);
+        __syncthreads();
+    }
+    __syncthreads();
+    for (int c = threadIdx.x; c < S; c += blockDim.x) qgrid[c] = q[c];
+    if (threadIdx.x == 0) {
+        status[0] = sweeps;
+        status[1] = converged ? 1 : 0;
+    }
+}
+
+// Project's divergence field as k2s_poisson_lds reads it (one thread per
+// element of dvs): div in the field type, times dx2 and dy2.
+template <class T>
+__global__ void k2s_div_skew(int nx, int ny, int P, int rp, const uint8_t* __restrict__ type, L3<T> w,
+                             T dx, T dy, double dx2, double dy2, double* __restrict__ dvs) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (P + kDvRows) * rp) return;
+    const int res = t / rp - kDvRows, i = t % rp;
+    int j = (res - i) % P - 1;
+    if (j < -1) j += P;
+    double v = __hiloint2double((int)kNotInner, 0);
+    if (i < nx && j >= 0 && j < ny) {
+        const int64_t c = (int64_t)i * ny + j;
+        if (type[c] == NODE_IN) {
+            const T* U = w.f[0];
+            const T* V = w.f[1];
+            const T dv = (U[c + ny] - U[c - ny]) / (2 * dx) + (V[c + 1] - V[c - 1]) / (2 * dy);
+            v = (double)dv * dx2 * dy2;
+        }
+    }
+    dvs[t] = v;
+}
+
+// q of the anti-diagonal layout over the whole grid for the gradient.
+template <class T>
+__global__ void k2s_undiag(int nx, int ny, int P, const T* __restrict__ qgrid, T* __restrict__ qf) {
+    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= (int64_t)nx * ny) return;
+    const int i = (int)(c / ny), j = (int)(c % ny);
+    qf[c] = qgrid[(int64_t)((i + j + 1) % P) * (nx + 2) + i + 1];
+}
+
 // q over the whole grid (zero outside the spans) for the gradient.
 template <class T>
 __global__ void k2s_unspan(int nx, int ny, const int32_t* __restrict__ spans,
@@ -856,6 +1201,12 @@ class Solver2D final : public ISolver2 {
     uint8_t* d_fspan = nullptr;
     int32_t* d_pstat = nullptr;
     int S = 0;
+    // k2s_poisson_lds (rl_P != 0: q fits the LDS): its P, the slice
+    // length, members, boundary wavefronts, boundary list pitch
+    int rl_P = 0, rl_rp = 0, rl_D = 0, rl_mw = 1, rl_bw = 0, rl_cpad = 0;
+    uint2* d_blist = nullptr;
+    double* d_dvs = nullptr;
+    T *d_qpad = nullptr, *d_qsave = nullptr;
     double ptol = 1e-2;            // POISSON_ERR_THRESHOLD (StableSolver2D.h:23)
     int64_t pcap = 1000000;        // the reference has no cap
     std::vector<int32_t> sweeps;   // relaxation sweeps of each project of the last step
@@ -974,6 +1325,64 @@ class Solver2D final : public ISolver2 {
         CMCX_HIP(hipMemcpyAsync(d_spans, sp.data(), sizeof(int32_t) * sp.size(), hipMemcpyHostToDevice, st));
         if (S) CMCX_HIP(hipMemcpyAsync(d_fspan, fl.data(), S, hipMemcpyHostToDevice, st));
         CMCX_HIP(hipStreamSynchronize(st));
+        build_fronts(t);
+    }
+
+    // Layout and boundary lists of k2s_poisson_lds, when its q fits the LDS and a
+    // cell's place in sweep order 16 bits.
+    void build_fronts(const uint8_t* t) {
+        const int rp = (nx + 63) / 64 * 64, smax = std::max(1, std::min(15, (1024 - 64) / rp));
+        int P = std::max(ny + 1, kPoisLag * smax);
+        if (nx > P) P = std::min(nx, (P + 63) / 64 * 64);
+        const int64_t cells = (int64_t)(nx + 2) * P;
+        if (cells * (int64_t)sizeof(T) + 3072 > 160 * 1024 || cells > 0xffff) return;
+        auto T_ = [&](int i, int j) -> int {
+            return (i < 0 || j < 0 || i >= nx || j >= ny) ? (int)NODE_OUT : t[(int64_t)i * ny + j];
+        };
+        std::vector<std::vector<uint2>> lists(P);
+        int cmax = 1;
+        for (int i = 0; i < nx; i++)
+            for (int j = 0; j < ny; j++) {
+                const int ty = T_(i, j), x = j + 1;
+                if (ty != NODE_BOUND && ty != NODE_VALVE) continue;
+                uint32_t w = kBValid | (uint32_t)(i * P + x);
+                if (T_(i - 1, j) == NODE_IN) w |= 1u << 16;
+                if (T_(i + 1, j) == NODE_IN) w |= 1u << 17;
+                if (T_(i, j - 1) == NODE_IN) w |= 1u << 18;
+                if (T_(i, j + 1) == NODE_IN) w |= 1u << 19;
+                auto& l = lists[(i + x) % P];
+                l.push_back(uint2{w, (uint32_t)i | (uint32_t)((i + x) / P) << 16});
+                cmax = std::max(cmax, (int)l.size());
+            }
+        // sweeps per slice as the row length allows; as many slices as leave the
+        // boundary wavefronts a lane for every boundary cell of a front (at
+        // least half of them otherwise)
+        int D = 0, bw = 1, mw = 1;
+        for (int sl = smax; sl >= std::max(1, smax / 2); sl--) {
+            const int room = 16 - sl * rp / 64;
+            mw = kPoisLag * 2 * sl <= P ? 2 : 1;
+            D = mw * sl;
+            bw = std::min(room, std::max((cmax * D + 63) / 64, 1));
+            if (64 * bw / D >= cmax) break;
+        }
+        const int epm = 64 * bw / D, cpad = (cmax + epm - 1) / epm * epm;
+        std::vector<uint2> bl((size_t)P * cpad, uint2{0, 0});
+        for (int q = 0; q < P; q++) std::copy(lists[q].begin(), lists[q].end(), bl.begin() + (size_t)q * cpad);
+        hipFree(d_blist);
+        d_blist = nullptr;
+        CMCX_HIP(hipMalloc((void**)&d_blist, sizeof(uint2) * bl.size()));
+        CMCX_HIP(hipMemcpy(d_blist, bl.data(), sizeof(uint2) * bl.size(), hipMemcpyHostToDevice));
+        if (!d_dvs) {
+            CMCX_HIP(hipMalloc((void**)&d_dvs, sizeof(double) * (P + kDvRows) * rp));
+            CMCX_HIP(hipMalloc((void**)&d_qpad, sizeof(T) * cells));
+            CMCX_HIP(hipMalloc((void**)&d_qsave, sizeof(T) * cells));
+        }
+        rl_P = P;
+        rl_rp = rp;
+        rl_D = D;
+        rl_mw = mw;
+        rl_bw = bw;
+        rl_cpad = cpad;
     }
 
     // Grid2D::Prepare(t) between steps (FluidSolver2D.cpp:131): new cell types,
@@ -1026,6 +1435,10 @@ class Solver2D final : public ISolver2 {
         hipFree(d_qf);
         hipFree(d_qspan);
         hipFree(d_save);
+        hipFree(d_blist);
+        hipFree(d_dvs);
+        hipFree(d_qpad);
+        hipFree(d_qsave);
         hipFree(d_doff);
         hipFree(d_spans);
         hipFree(d_fspan);
@@ -1216,10 +1629,15 @@ class Solver2D final : public ISolver2 {
     // StableSolver2D::Project (StableSolver2D.cpp:83-165): w -> next on NODE_IN.
     // Returns false when the relaxation reached the sweep cap.
     bool project() {
-        hipLaunchKernelGGL((k2s_div<T>), dim3(blocks2(N)), dim3(kBS2), 0, st, nx, ny, d_type, nw,
-                           (T)prm.dx, (T)prm.dy, d_doff, d_dv);
-        CMCX_LAUNCH_CHECK();
         const double dx2 = prm.dx * prm.dx, dy2 = prm.dy * prm.dy, rcp = 0.5 / (dx2 + dy2);
+        const bool fronts = rl_P != 0;
+        if (fronts)
+            hipLaunchKernelGGL((k2s_div_skew<T>), dim3(blocks2((int64_t)(rl_P + kDvRows) * rl_rp)), dim3(kBS2), 0,
+                               st, nx, ny, rl_P, rl_rp, d_type, nw, (T)prm.dx, (T)prm.dy, dx2, dy2, d_dvs);
+        else
+            hipLaunchKernelGGL((k2s_div<T>), dim3(blocks2(N)), dim3(kBS2), 0, st, nx, ny, d_type, nw,
+                               (T)prm.dx, (T)prm.dy, d_doff, d_dv);
+        CMCX_LAUNCH_CHECK();
         const int rp = std::max(64, (nx + 63) / 64 * 64);  // threads per set
         const size_t lds = (size_t)S * sizeof(T) + (size_t)S;
         const bool in_lds = lds + 2048 <= 160 * 1024;
@@ -1227,7 +1645,14 @@ class Solver2D final : public ISolver2 {
         bool done = false;
         for (int resume = 0; !done && total < pcap; resume = 1) {
             const int chunk = (int)std::min<int64_t>(kPoisChunk, pcap - total);
-            if (in_lds) launch_poisson_for<true>(rp, lds, dx2, dy2, rcp, chunk, resume);
+            if (fronts) {
+                auto kern = rl_mw == 2 ? k2s_poisson_lds<T, 2> : k2s_poisson_lds<T, 1>;
+                hipLaunchKernelGGL(kern, dim3(1), dim3(rl_D / rl_mw * rl_rp + 64 * rl_bw),
+                                   sizeof(T) * (size_t)(nx + 2) * rl_P, st, nx, rl_P, rl_rp, rl_D, rl_bw,
+                                   rl_cpad, d_blist, d_dvs, d_qpad, d_qsave, dx2, dy2, rcp, ptol, chunk,
+                                   resume, d_pstat);
+                CMCX_LAUNCH_CHECK();
+            } else if (in_lds) launch_poisson_for<true>(rp, lds, dx2, dy2, rcp, chunk, resume);
             else launch_poisson_for<false>(rp, 0, dx2, dy2, rcp, chunk, resume);
             int32_t h[2];
             CMCX_HIP(hipMemcpyAsync(h, d_pstat, sizeof(h), hipMemcpyDeviceToHost, st));
@@ -1237,7 +1662,9 @@ class Solver2D final : public ISolver2 {
         }
         sweeps.push_back((int32_t)std::min<int64_t>(total, INT32_MAX));
         if (!done) return false;
-        hipLaunchKernelGGL((k2s_unspan<T>), dim3(blocks2(N)), dim3(kBS2), 0, st, nx, ny, d_spans, d_qspan,
+        if (fronts)
+            hipLaunchKernelGGL((k2s_undiag<T>), dim3(blocks2(N)), dim3(kBS2), 0, st, nx, ny, rl_P, d_qpad, d_qf);
+        else hipLaunchKernelGGL((k2s_unspan<T>), dim3(blocks2(N)), dim3(kBS2), 0, st, nx, ny, d_spans, d_qspan,
                            d_qf);
         hipLaunchKernelGGL((k2s_grad<T>), dim3(blocks2(N)), dim3(kBS2), 0, st, nx, ny, d_type, nw, d_qf,
                            (T)prm.dx, (T)prm.dy, next);
