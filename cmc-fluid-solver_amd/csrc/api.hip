@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <array>
 #include <cmath>
+#include <initializer_list>
 #include <map>
 #include <cstring>
 #include <memory>
@@ -81,6 +82,7 @@ struct Grid {
     SegList segs[3];
     int free_shared = 0;      // axes with a BC_FREE node shared by two segments
     double err = 0.0;         // divergence error of the last evaluation
+    bool has_out = false;     // holds NODE_OUT nodes
 };
 
 template <class T>
@@ -154,6 +156,11 @@ class Solver final : public ISolver {
     std::vector<uint8_t> out_fill;
     T* keep_buf = nullptr;
     Layer4<T> out_keep{};
+    // resampled output nodes on their way to the host (T, then u, v, w), at most
+    // kOutChunk of them
+    static constexpr int64_t kOutChunk = 1 << 20;
+    double* out_buf = nullptr;
+    int64_t out_cap = 0;
     // HIP graphs of whole steps, per (boundary fill, dt, G, L, state buffer)
     bool graph_mode = false;
     // (with the boundary-sync mode the sweeps were captured with)
@@ -223,6 +230,7 @@ class Solver final : public ISolver {
             const cmcx_domain* d = &doms[i];
             const int64_t o = grids[i].off, N = grids[i].g.N;
             std::memcpy(&h_type[o], d->type, N);
+            grids[i].has_out = std::memchr(d->type, NODE_OUT, N) != nullptr;
             std::memcpy(&h_bcv[o], d->bc_vel, N);
             std::memcpy(&h_bct[o], d->bc_temp, N);
             const double* src[4] = {d->v[0], d->v[1], d->v[2], d->T};
@@ -334,6 +342,7 @@ class Solver final : public ISolver {
         for (auto* p : d_g) hipFree(p);
         hipFree(buf);
         hipFree(keep_buf);
+        hipFree(out_buf);
         for (auto& G : grids)
             for (auto& s : G.segs) hipFree(s.d);
         hipFree(scratch);
@@ -830,11 +839,35 @@ class Solver final : public ISolver {
         return CMCX_OK;
     }
 
+    // Whether a kernel of this device may write every (non-null) address as
+    // elements of the field type; other memory is left to the runtime's copies.
+    static bool on_this_device(std::initializer_list<const void*> ptrs) {
+        int dev = -1;
+        if (hipGetDevice(&dev) != hipSuccess) return false;
+        for (const void* q : ptrs) {
+            if (!q) continue;
+            hipPointerAttribute_t a;
+            if (hipPointerGetAttributes(&a, q) != hipSuccess) {
+                (void)hipGetLastError();  // not an address the runtime knows
+                return false;
+            }
+            if (a.type != hipMemoryTypeDevice || a.device != dev || (uintptr_t)q % sizeof(T)) return false;
+        }
+        return true;
+    }
+
     int get_fields(void* u, void* v, void* w, void* p, void* Tt, bool device) override {
         const Grid& Gr = G();
         const int64_t N = Gr.g.N, o = Gr.off;
         hipMemcpyKind k = device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
         void* dst[4] = {u, v, w, Tt};
+        if (device && on_this_device({u, v, w, p, Tt})) {
+            Layer4<T> to;
+            for (int f = 0; f < 4; f++) to.f[f] = (T*)dst[f];
+            launch_read_state<T>(shifted(cur, o), to, (T*)p, (T)Gr.prm.v_T, N, st);
+            CMCX_HIP(hipStreamSynchronize(st));
+            return CMCX_OK;
+        }
         for (int f = 0; f < 4; f++)
             if (dst[f]) CMCX_HIP(hipMemcpyAsync(dst[f], cur.f[f] + o, sizeof(T) * N, k, st));
         if (p) {
@@ -884,29 +917,30 @@ class Solver final : public ISolver {
         if (oy == 0) oy = g.ny;
         if (oz == 0) oz = g.nz;
         // Solver3D::GetLayer: next->Clear(grid, NODE_OUT, 99999, ...) then FilterToArrays
-        T miss = (T)99999.0f;
-        launch_fill_typed<T>(g, d_type + Gr.off, NODE_OUT, shifted(next, Gr.off), miss, miss, miss, miss, st);
-        out_fill[sel] |= (uint8_t)(1 << state_buffer(next));
-        const int64_t N = g.N;
-        std::vector<T> h[4];
-        for (int f = 0; f < 4; f++) {
-            h[f].resize(N);
-            CMCX_HIP(hipMemcpyAsync(h[f].data(), next.f[f] + Gr.off, sizeof(T) * N,
-                                    hipMemcpyDeviceToHost, st));
+        // (a grid without NODE_OUT nodes has nothing to clear, and its two state
+        // buffers never come to disagree, see out_fill)
+        if (Gr.has_out) {
+            const T miss = (T)99999.0f;
+            launch_fill_typed<T>(g, d_type + Gr.off, NODE_OUT, shifted(next, Gr.off), miss, miss, miss, miss, st);
+            out_fill[sel] |= (uint8_t)(1 << state_buffer(next));
+        }
+        // resampled on the device, kOutChunk nodes at a time
+        const int64_t n = (int64_t)ox * oy * oz, cap = std::min(n, kOutChunk);
+        if (cap > out_cap) {
+            hipFree(out_buf);
+            out_buf = nullptr;
+            out_cap = 0;
+            CMCX_HIP(hipMalloc((void**)&out_buf, (sizeof(double) + 3 * sizeof(T)) * cap));
+            out_cap = cap;
+        }
+        T* const d_vel = reinterpret_cast<T*>(out_buf + cap);
+        for (int64_t first = 0; first < n; first += cap) {
+            const int64_t m = std::min(cap, n - first);
+            launch_resample<T>(g, shifted(next, Gr.off), ox, oy, oz, first, m, d_vel, out_buf, st);
+            CMCX_HIP(hipMemcpyAsync((T*)vel + 3 * first, d_vel, 3 * sizeof(T) * m, hipMemcpyDeviceToHost, st));
+            CMCX_HIP(hipMemcpyAsync(Tout + first, out_buf, sizeof(double) * m, hipMemcpyDeviceToHost, st));
         }
         CMCX_HIP(hipStreamSynchronize(st));
-        T* V = (T*)vel;
-        for (int i = 0; i < ox; i++)
-            for (int j = 0; j < oy; j++)
-                for (int k = 0; k < oz; k++) {
-                    int x = i * g.nx / ox, y = j * g.ny / oy, z = k * g.nz / oz;
-                    int64_t src = x * g.sx + y * g.sy + z;
-                    int64_t ind = ((int64_t)i * oy + j) * oz + k;
-                    V[3 * ind + 0] = h[0][src];
-                    V[3 * ind + 1] = h[1][src];
-                    V[3 * ind + 2] = h[2][src];
-                    Tout[ind] = (double)h[3][src];
-                }
         return CMCX_OK;
     }
 

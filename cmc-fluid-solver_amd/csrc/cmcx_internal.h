@@ -221,6 +221,13 @@ int div_partials();
 template <class T>
 void launch_div_error(const Geom& g, const uint8_t* type, Layer4<T> L, T hx, T hy, T hz,
                       double* d_acc, double* d_part, hipStream_t st);
+// u, v, w, T of a state (entries of dst, null = none) and p = v_T T (null = none).
+template <class T>
+void launch_read_state(Layer4<T> src, Layer4<T> dst, T* p, T v_T, int64_t n, hipStream_t st);
+// Nodes [first, first + n) of a layer resampled to (ox, oy, oz): vel (3 per node), T.
+template <class T>
+void launch_resample(const Geom& g, Layer4<T> L, int ox, int oy, int oz, int64_t first, int64_t n,
+                     T* vel, double* Tout, hipStream_t st);
 template <class T>
 void launch_scale(const T* src, T* dst, T a, int64_t n, hipStream_t st);
 template <class T>

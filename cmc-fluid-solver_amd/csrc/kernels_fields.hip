@@ -102,6 +102,54 @@ __global__ void copy4_kernel(int64_t n, Layer4<T> dst, Layer4<T> src) {
     for (int f = 0; f < 4; f++) dst.f[f][i] = src.f[f][i];
 }
 
+// The state (u, v, w, T, and p = v_T T) into a program's arrays, each optional,
+// in one launch: 16-byte vectors at any element address.  Five copies of one
+// launch each took about 25 us on a small grid, almost all of it launches.
+template <class T>
+__global__ void __launch_bounds__(kBS) read_state_kernel(int64_t n, Layer4<T> src, Layer4<T> dst,
+                                                         T* __restrict__ p, T v_T) {
+    constexpr int W = 16 / (int)sizeof(T);
+    typedef T V __attribute__((ext_vector_type(W), aligned(sizeof(T))));
+    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * W;
+    if (i + W <= n) {
+        V v[4];
+#pragma unroll
+        for (int f = 0; f < 4; f++) v[f] = *reinterpret_cast<const V*>(src.f[f] + i);
+#pragma unroll
+        for (int f = 0; f < 4; f++)
+            if (dst.f[f]) *reinterpret_cast<V*>(dst.f[f] + i) = v[f];
+        if (p) *reinterpret_cast<V*>(p + i) = v[3] * v_T;
+    } else {
+        for (int64_t k = i; k < n; k++) {
+#pragma unroll
+            for (int f = 0; f < 4; f++)
+                if (dst.f[f]) dst.f[f][k] = src.f[f][k];
+            if (p) p[k] = src.f[3][k] * v_T;
+        }
+    }
+}
+
+// FilterToArrays (TimeLayer3D.h): output nodes [first, first + n) of a layer
+// resampled to (ox, oy, oz) by nearest index, vel 3 values and T a double per
+// node.  Gathered here, only the output nodes cross to the host: a 128 x 96 x
+// 112 FP32 layer resampled to 50^3 moves 2.5 MB instead of the layer's 22 MB,
+// which the host gathered from.
+template <class T>
+__global__ void __launch_bounds__(kBS) resample_kernel(Geom g, Layer4<T> L, int ox, int oy, int oz,
+                                                       int64_t first, int64_t n,
+                                                       T* __restrict__ vel,
+                                                       double* __restrict__ Tout) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= n) return;
+    const int64_t q = first + t, ij = q / oz;
+    const int64_t i = ij / oy, j = ij - i * oy, k = q - ij * oz;
+    const int64_t src = (i * g.nx / ox) * g.sx + (j * g.ny / oy) * g.sy + k * g.nz / oz;
+    vel[3 * t] = L.f[0][src];
+    vel[3 * t + 1] = L.f[1][src];
+    vel[3 * t + 2] = L.f[2][src];
+    Tout[t] = (double)L.f[3][src];
+}
+
 // EvalDivError (TimeLayer3D.h:595-641): per NODE_IN node with i < nx-1, j < ny-1,
 // k < nz-1, |flux divergence| of the dual cell; field-type sums, double result.
 // Grid-stride loop, one (sum, count) partial per block, summed in block order by
@@ -288,6 +336,22 @@ void launch_div_error(const Geom& g, const uint8_t* type, Layer4<T> L, T hx, T h
 }
 
 template <class T>
+void launch_read_state(Layer4<T> src, Layer4<T> dst, T* p, T v_T, int64_t n, hipStream_t st) {
+    constexpr int W = 16 / (int)sizeof(T);
+    hipLaunchKernelGGL((read_state_kernel<T>), dim3(blocks_for(n, kBS * W)), dim3(kBS), 0, st, n, src,
+                       dst, p, v_T);
+    CMCX_LAUNCH_CHECK();
+}
+
+template <class T>
+void launch_resample(const Geom& g, Layer4<T> L, int ox, int oy, int oz, int64_t first, int64_t n,
+                     T* vel, double* Tout, hipStream_t st) {
+    hipLaunchKernelGGL((resample_kernel<T>), dim3(blocks_for(n)), dim3(kBS), 0, st, g, L, ox, oy, oz,
+                       first, n, vel, Tout);
+    CMCX_LAUNCH_CHECK();
+}
+
+template <class T>
 void launch_scale(const T* src, T* dst, T a, int64_t n, hipStream_t st) {
     hipLaunchKernelGGL((scale_kernel<T>), dim3(blocks_for(n)), dim3(kBS), 0, st, src, dst, a, n);
     CMCX_LAUNCH_CHECK();
@@ -338,6 +402,9 @@ void launch_mask_check(const Geom& g, const uint8_t* type, unsigned long long* d
                                       Layer4<T>, Layer4<T>, hipStream_t);                          \
     template void launch_div_error<T>(const Geom&, const uint8_t*, Layer4<T>, T, T, T, double*,    \
                                       double*, hipStream_t);                                       \
+    template void launch_read_state<T>(Layer4<T>, Layer4<T>, T*, T, int64_t, hipStream_t);         \
+    template void launch_resample<T>(const Geom&, Layer4<T>, int, int, int, int64_t, int64_t, T*,  \
+                                     double*, hipStream_t);                                        \
     template void launch_scale<T>(const T*, T*, T, int64_t, hipStream_t);                          \
     template void launch_convert_from_f64<T>(const double*, T*, int64_t, hipStream_t);             \
     template void launch_copy_typed<T>(const Geom&, const uint8_t*, int, Layer4<T>, Layer4<T>,     \
