@@ -120,11 +120,7 @@ class Solver final : public ISolver {
     size_t scratch_elems = 0;
     FusedWork work[3][kFusedVariants];
     InstDesc<T>* d_desc = nullptr;
-    // fused kernel variant per axis (autotuned).  Z lines of more than 128 nodes
-    // start out spread over 64 lanes: 8 rows per lane take over 200 registers
-    // (FP32) or 400 (FP64).  Measured per sweep, 32 against 64 lanes: FP32 192^3
-    // 96 / 82 us, 256^3 200 / 189; FP64 160^3 180 / 125, 192 x 192 x 256 336 /
-    // 242; at 128 nodes 32 lanes win (FP64 256 x 256 x 128 203 / 225).
+    // fused kernel variant per axis (fused_default_variant, or autotuned)
     int variant[3] = {0, 0, 0};
     double* d_acc = nullptr;     // 2 doubles per grid
     double* d_part = nullptr;
@@ -217,8 +213,11 @@ class Solver final : public ISolver {
             G.off = off;
             off += (G.g.N + 63) / 64 * 64;  // 256-byte aligned grids
         }
-        for (const Grid& Gr : grids)
-            if (Gr.g.nz > 128) variant[AX_Z] = 4;
+        {
+            std::vector<Geom> gs;
+            for (const Grid& Gr : grids) gs.push_back(Gr.g);
+            for (int a = 0; a < 3; a++) variant[a] = fused_default_variant<T>(gs, a);
+        }
         NT = off;
         if (NT > ((int64_t)1 << 31) - 1) throw std::string("grids too large (total node count must fit in int32)");
         h_type.assign(NT, (uint8_t)NODE_OUT);  // padding between grids: never read

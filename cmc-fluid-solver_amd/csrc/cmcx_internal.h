@@ -145,6 +145,9 @@ int strided_chunk_rows(int variant);
 // Strided variant v usable for lines of n nodes.
 template <class T>
 bool fused_variant_ok(int n, int v);
+// Variant that a set of grids starts out with on an axis (until autotuned).
+template <class T>
+int fused_default_variant(const std::vector<Geom>& gs, int axis);
 // Node flags of the fused kernels: type | kFlagFreeVel | kFlagFreeT (0 on NODE_IN).
 constexpr uint8_t kFlagFreeVel = 4, kFlagFreeT = 8;
 void build_node_flags(const uint8_t* t, const uint8_t* bv, const uint8_t* bt, int64_t n,

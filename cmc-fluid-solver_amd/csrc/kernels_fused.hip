@@ -856,6 +856,38 @@ bool fused_variant_ok(int n, int v) {
     return strided_variant_fits<T>(n, v);
 }
 
+// Z: lines of more than 128 nodes start out spread over 64 lanes: 8 rows per
+// lane take over 200 registers (FP32) or 400 (FP64).  Measured per sweep, 32
+// against 64 lanes: FP32 192^3 96 / 82 us, 256^3 200 / 189; FP64 160^3 180 /
+// 125, 192 x 192 x 256 336 / 242.
+// FP64 lines of 96 to 128 nodes do with 4 rows less per lane too, registers
+// capped and the Picard layer parked (128^3 step 650 / 635 us, 128 x 96 x 112 409
+// / 402); shorter ones lose (64^3 +5 %).
+// X and Y: up to 64 tiles of 128-byte rows leave most of the 256 CUs idle, so
+// lines of at most 64 nodes take 32-byte tiles of 4-row chunks (24^3 and 32^3:
+// FP32 step 80 / 73 us, FP64 101 / 92).  Otherwise 128-byte tiles; the Picard
+// layer is parked in LDS for the merge once its four fields are 8 MiB, a quarter
+// of the chip's L2: the second read of a smaller one hits there (64^3 FP32: 112 us
+// read again, 115 parked), that of a larger one goes further out (FP32 128^3
+// 295 / 261 us, 250 x 203 x 187 1987 / 1908; FP64 128^3 690 / 650).
+template <class T>
+int fused_default_variant(const std::vector<Geom>& gs, int axis) {
+    int n = 0;
+    int64_t tiles = 0, bytes = 0;  // tiles of 128-byte rows, bytes of four fields
+    for (const Geom& g : gs) {
+        bytes += 4 * g.N * (int64_t)sizeof(T);
+        n = std::max(n, axis == AX_Z ? g.nz : axis == AX_X ? g.nx : g.ny);
+        const int lpg = variant_lpg<T>(0);
+        tiles += (int64_t)(axis == AX_X ? g.ny : g.nx) * ((g.nz + lpg - 1) / lpg);
+    }
+    if (axis == AX_Z) {
+        if (n > 128) return 4;
+        return sizeof(T) == 8 && n >= 96 ? 7 : 0;
+    }
+    if (n <= 64 && tiles <= 64) return 5;
+    return bytes >= (8 << 20) && strided_variant_fits<T>(n, 6) ? 6 : 0;
+}
+
 template <class T>
 void launch_fused_sweep(const InstDesc<T>* insts, T three_dt, int axis, const FusedWork& w,
                         const uint8_t* tflags, const T* const* gval, Layer4<T> in, Layer4<T> tin,
@@ -1120,6 +1152,8 @@ template bool fused_supported<float>(const Geom&);
 template bool fused_supported<double>(const Geom&);
 template bool fused_variant_ok<float>(int, int);
 template bool fused_variant_ok<double>(int, int);
+template int fused_default_variant<float>(const std::vector<Geom>&, int);
+template int fused_default_variant<double>(const std::vector<Geom>&, int);
 template int strided_lpg<float>(int);
 template int strided_lpg<double>(int);
 template int strided_chunk_rows<float>(int);
