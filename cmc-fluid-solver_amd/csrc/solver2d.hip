@@ -31,8 +31,10 @@
 #pragma clang fp contract(off)
 
 #include "cmcx_internal.h"
+#include "line_solve.h"
 
 #include <algorithm>
+#include <cmath>
 #include <memory>
 #include <vector>
 
@@ -400,6 +402,232 @@ __global__ void __launch_bounds__(kSweepLdsThreads) k2_sweep_lds(
             x = bd_[k] - bc_[k] * x;
             put(t - k, x, bf_[k]);
         }
+}
+
+// The same solve with a line's recurrences cut into chunks of CL rows, a lane
+// each, and every value still the serial one's, bit for bit.  A row's c', d' (and
+// x) depend on the rows before it less and less: an error in them shrinks by
+// about |c'| per row, until rounding leaves none of it.  So each lane starts some
+// rows early from zero: `wa` rows with an approximate reciprocal bring it within
+// a few bits, kChunkExact rows with the exact operations to the value itself,
+// as a rule.  Then it compares the values that it entered its chunk with to the
+// lane before's at its end, and where they differ takes those and runs its chunk
+// again, until no lane differs: then every chunk continues its predecessor's
+// exactly, and the first one started the line.  One more chunk is settled each
+// time, so it ends whatever the rows (infinite and NaN values too).  Back
+// substitution likewise from the line's end (`wb` rows early).
+// k2_sweep_lds is a chain of two FP64 divisions per row, some 220 ns each: lines
+// of 256 rows took 58 us there and of 128 rows 31, and take 18 and 14 here (build
+// of the rows 3 to 6, elimination 2 to 6, back substitution 1 to 4 us).
+constexpr int kChunkExact = 12;
+constexpr int kChunkMaxRows = 64 * 8;   // rows of a line at most
+constexpr int kChunkMaxSystems = 2048;  // of one sweep at most: more of them fill the chip line by line
+
+__device__ __forceinline__ float approx_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
+__device__ __forceinline__ double approx_rcp(double x) {
+    const double r = __builtin_amdgcn_rcp(x);
+    return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+}
+__device__ __forceinline__ bool same_bits(float a, float b) { return __float_as_uint(a) == __float_as_uint(b); }
+__device__ __forceinline__ bool same_bits(double a, double b) {
+    return __double_as_longlong(a) == __double_as_longlong(b);
+}
+
+// Rows of a system in LDS: `w` = wa + kChunkExact before its first, its own up to
+// whole chunks, wb after them, and one of padding per chunk (the lanes' rows are
+// then on different banks); the rows that are not its own (a = 0, b = 1, c = d
+// = 0) leave zero, so that the early starts need no conditions.
+__host__ __device__ constexpr int chunk_rows(int nmax, int w, int wb, int cl) { return w + (nmax + cl - 1) / cl * cl + wb; }
+__host__ __device__ constexpr int chunk_pitch(int rows, int cl) { return rows + rows / cl + 1; }
+
+template <class T, bool DIRX, int CL>
+__global__ void __launch_bounds__(kSweepLdsThreads) k2_sweep_chunks(
+    int nsys, int spw, int nmax, const Sys2* __restrict__ sys, int nx, int ny,
+    const uint8_t* __restrict__ type, const uint8_t* __restrict__ bc, L3<T> g, L3<T> lc,
+    L3<T> tl, L3<T> out, L3<T> lt, int mode, P2 prm, int wa, int wb) {
+    extern __shared__ __align__(16) char smem2[];
+    Row4<T>* const rw = reinterpret_cast<Row4<T>*>(smem2);
+    const int w = wa + kChunkExact, rows = chunk_rows(nmax, w, wb, CL), pitch = chunk_pitch(rows, CL);
+    const int var = blockIdx.y;
+    // neighbouring lines, which share cache lines, on one XCD
+    const int s0 = (int)lsolve::xcd_remap(blockIdx.x, gridDim.x) * spw;
+    const int nloc = min(spw, nsys - s0);
+    auto cell = [&](const Sys2& q, int t) -> int64_t {
+        return DIRX ? (int64_t)(q.a0 + t) * ny + q.a1 : (int64_t)q.a0 * ny + q.a1 + t;
+    };
+    // consecutive threads on neighbouring cells
+    for (int e = threadIdx.x; e < spw * rows; e += blockDim.x) {
+        const int sl = DIRX ? e % spw : e / rows, u = DIRX ? e / spw : e % rows;
+        if (sl >= nloc) continue;
+        const Sys2 q = sys[s0 + sl];
+        const int n = DIRX ? q.b - q.a0 + 1 : q.b - q.a1 + 1, t = u - w;
+        Row4<T> r;
+        r.a = r.c = r.d = 0;
+        r.b = 1;
+        if (t >= 0 && t < n) row2<T, DIRX>(t, n, var, cell(q, t), ny, bc, g, lc, tl, prm, r.a, r.b, r.c, r.d);
+        rw[sl * pitch + u + u / CL] = r;
+    }
+    __syncthreads();
+
+    for (int sl = threadIdx.x >> 6; sl < nloc; sl += kSweepLdsThreads / 64) {
+        const Sys2 q = sys[s0 + sl];
+        const int n = DIRX ? q.b - q.a0 + 1 : q.b - q.a1 + 1;
+        const int lane = threadIdx.x & 63, last = (n - 1) / CL;  // lanes past the last chunk repeat it
+        const bool on = lane <= last;
+        const int s = min(lane, last) * CL;  // first row of the lane's chunk
+        // row s - w + i, i uniform
+        Row4<T>* const my = rw + sl * pitch + s + s / CL;
+        auto at = [&](int i) -> Row4<T>& { return my[i + i / CL]; };
+        T cp = 0, dp = 0;
+        Row4<T> A[4], B[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) A[k] = at(k);
+        for (int i = 0; i < wa; i += 4) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) B[k] = at(i + 4 + k);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const T iv = approx_rcp(__builtin_fma(-A[k].a, cp, A[k].b));
+                cp = A[k].c * iv;
+                dp = __builtin_fma(-A[k].a, dp, A[k].d) * iv;
+            }
+#pragma unroll
+            for (int k = 0; k < 4; k++) A[k] = B[k];
+        }
+        auto step = [&](const Row4<T>& r) {
+            const T den = r.b - r.a * cp;
+            cp = r.c / den;
+            dp = (r.d - dp * r.a) / den;
+        };
+#pragma unroll
+        for (int i = 0; i < kChunkExact; i += 4) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) B[k] = at(wa + i + 4 + k);
+#pragma unroll
+            for (int k = 0; k < 4; k++) step(A[k]);
+#pragma unroll
+            for (int k = 0; k < 4; k++) A[k] = B[k];
+        }
+        Row4<T> own[CL];
+#pragma unroll
+        for (int k = 0; k < CL; k++) own[k] = k < 4 ? A[k] : at(w + k);
+        // Row 0 takes no values from before it (a = 0).
+        T cin = s == 0 ? (T)0 : cp, din = s == 0 ? (T)0 : dp, cv[CL], dv[CL], den[CL];
+        bool quick = true;
+        for (;;) {
+            cp = cin;
+            dp = din;
+#pragma unroll
+            for (int k = 0; k < CL; k++) {
+                den[k] = own[k].b - own[k].a * cp;
+                cp = own[k].c / den[k];
+                dp = (own[k].d - dp * own[k].a) / den[k];
+                cv[k] = cp;
+                dv[k] = dp;
+            }
+            T pc = lsolve::lane_prev(cp), pd = lsolve::lane_prev(dp);
+            bool bad = on && lane > 0 && !(same_bits(pc, cin) && same_bits(pd, din));
+            if (!__any(bad)) break;
+            const bool settled = !__any(on && lane > 0 && !same_bits(pc, cin));
+            cin = bad ? pc : cin;
+            din = bad ? pd : din;
+            // Once c' is settled, d' goes on with its pivots' reciprocals and one
+            // correction, a quotient as a rule, until no lane differs; the pass
+            // above has the last word.  For lines where d' only decays (no
+            // right-hand side left), whose bits depend on every row before: a
+            // pass is then one chunk's progress, of 26 instructions instead of 200.
+            if (quick && settled) {
+                quick = false;
+                T rden[CL];
+#pragma unroll
+                for (int k = 0; k < CL; k++) rden[k] = (T)1 / den[k];
+                for (int pass = 0; pass < 64; pass++) {
+                    dp = din;
+#pragma unroll
+                    for (int k = 0; k < CL; k++) {
+                        const T num = own[k].d - dp * own[k].a, v = num * rden[k];
+                        dp = __builtin_fma(__builtin_fma(-den[k], v, num), rden[k], v);
+                    }
+                    pd = lsolve::lane_prev(dp);
+                    bad = on && lane > 0 && !same_bits(pd, din);
+                    if (!__any(bad)) break;
+                    din = bad ? pd : din;
+                }
+            }
+        }
+        // (the last row's x is its d'; rows past the end leave zero)
+#pragma unroll
+        for (int k = 0; k < CL; k++) {
+            if (s + k >= n - 1) cv[k] = 0;
+            if (s + k >= n) dv[k] = 0;
+        }
+        // c', d' over c, d: every lane of the system's wavefront has read its rows
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int k = 0; k < CL; k++)
+            if (on && s + k < n) {
+                at(w + k).c = cv[k];
+                at(w + k).d = dv[k];
+            }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        // x of the row after the chunk
+        T x = 0, C[4], D[4];
+        const int top = w + CL + wb - 1;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            C[k] = at(top - k).c;
+            D[k] = at(top - k).d;
+        }
+        for (int i = 0; i < wb; i += 4) {
+            T nc[4], nd[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                nc[k] = at(top - i - 4 - k).c;
+                nd[k] = at(top - i - 4 - k).d;
+            }
+#pragma unroll
+            for (int k = 0; k < 4; k++) x = D[k] - C[k] * x;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                C[k] = nc[k];
+                D[k] = nd[k];
+            }
+        }
+        T xin = x, xs[CL];
+        for (;;) {
+            x = xin;
+#pragma unroll
+            for (int k = CL - 1; k >= 0; k--) {
+                x = dv[k] - cv[k] * x;
+                xs[k] = x;
+            }
+            const T xn = lsolve::lane_next(xs[0]);
+            const bool bad = lane < last && !same_bits(xn, xin);
+            if (!__any(bad)) break;
+            xin = bad ? xn : xin;
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int k = 0; k < CL; k++)
+            if (on && s + k < n) at(w + k).d = xs[k];
+    }
+    __syncthreads();
+    T* const o1 = out.f[var];
+    T* const o2 = mode == 1 ? lt.f[var] : o1;
+    for (int e = threadIdx.x; e < spw * nmax; e += blockDim.x) {
+        const int sl = DIRX ? e % spw : e / nmax, t = DIRX ? e / spw : e % nmax;
+        if (sl >= nloc) continue;
+        const Sys2 q = sys[s0 + sl];
+        if (t >= (DIRX ? q.b - q.a0 + 1 : q.b - q.a1 + 1)) continue;
+        const int64_t ct = cell(q, t);
+        const int i = DIRX ? q.a0 + t : q.a0, j = DIRX ? q.a1 : q.a1 + t;
+        if (mode == 0 || (type[ct] == NODE_IN && i < nx - 1 && j < ny - 1)) {
+            const int u = t + w;
+            const T v = rw[sl * pitch + u + u / CL].d;
+            o1[ct] = v;
+            o2[ct] = v;
+        }
+    }
 }
 
 // TimeLayer2D::EvalDivError: per-block partial sums of |tx + ty| in the field
@@ -1518,10 +1746,45 @@ class Solver2D final : public ISolver2 {
         return per <= 150 * 1024 ? spw : 0;
     }
 
+    // Rows after which an error in c', d' or x has shrunk below the rounding of a
+    // line's values, from the viscous part of the rows (its |c'| for constant
+    // rows): the length of the chunks' early starts.  0: lines are solved
+    // serially (k2_sweep_lds): too many rows or systems, or the early starts
+    // (about 0.3 of a serial row each) and the exact ones cost most of the line.
+    int early_rows(bool dirx) const {
+        const int n = dirx ? nrows : ncols, nmax = dirx ? rows_nmax : cols_nmax;
+        if (nmax > kChunkMaxRows || 3 * n > kChunkMaxSystems) return 0;
+        const double h = dirx ? prm.dx : prm.dy, vis = std::max(prm.v_vis, prm.t_vis) / (h * h);
+        const double b = 1.0 / prm.dt + 2 * vis;
+        double w = 0;
+        if (vis > 0) {
+            const double c = (b - std::sqrt(b * b - 4 * vis * vis)) / (2 * vis);
+            w = (sizeof(T) == 8 ? 56 : 27) / -std::log2(c);
+        }
+        const double rows = w + 4;
+        if (!(rows >= 4) || 0.3 * std::min<double>(rows, nmax) + kChunkExact + 4 > 0.8 * nmax) return 0;
+        return (int)std::min<double>(rows, nmax);
+    }
+
     // mode 1: k2_sweep_lds writes lt and out on the NODE_IN rows (a direction
     // with one inner iteration), else the solution into out
     void sweep_lds(bool dirx, int spw, int mode, L3<T> lc, L3<T> tlc, L3<T> out, L3<T> lt) {
         const int n = dirx ? nrows : ncols, nmax = dirx ? rows_nmax : cols_nmax;
+        if (const int early = early_rows(dirx)) {
+            // a wavefront per system
+            const int cl = nmax <= 64 * 4 ? 4 : 8;
+            const int w = (std::max(early, kChunkExact + 4) + cl - 1) / cl * cl, wa = w - kChunkExact;
+            const int wb = (early + 3) / 4 * 4, pitch = chunk_pitch(chunk_rows(nmax, w, wb, cl), cl);
+            int per = std::min(spw, kSweepLdsThreads / 64);
+            while (per > 1 && per * pitch * sizeof(Row4<T>) > 150 * 1024) per /= 2;
+            auto kern = dirx ? (cl == 4 ? k2_sweep_chunks<T, true, 4> : k2_sweep_chunks<T, true, 8>)
+                             : (cl == 4 ? k2_sweep_chunks<T, false, 4> : k2_sweep_chunks<T, false, 8>);
+            hipLaunchKernelGGL(kern, dim3((unsigned)((n + per - 1) / per), 3), dim3(kSweepLdsThreads),
+                               (size_t)per * pitch * sizeof(Row4<T>), st, n, per, nmax, dirx ? d_rows : d_cols, nx, ny, d_type,
+                               d_bc, g, lc, tlc, out, lt, mode, prm, wa, wb);
+            CMCX_LAUNCH_CHECK();
+            return;
+        }
         const size_t lds = (size_t)spw * nmax * (sizeof(Row4<T>) + 1);
         const dim3 grid((unsigned)((n + spw - 1) / spw), 3);
         if (dirx)
