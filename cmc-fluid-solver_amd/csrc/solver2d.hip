@@ -71,13 +71,10 @@ __global__ void k2_copy(int nx, int ny, const uint8_t* __restrict__ type, int ma
     for (int f = 0; f < 3; f++) dst.f[f][q] = merge ? (dst.f[f][q] + src.f[f][q]) / 2 : src.f[f][q];
 }
 
-// Fused copies of the one-iteration path, on nodes (i < nx-1, j < ny-1) as
-// k2_copy.  k2_fan: d0..d3 <- src (the step's copies of the state, with the
-// first X direction's copy of the Picard layer).  k2_merge_fan: temp <- next
-// on NODE_IN (merge: (temp + next) / 2), then tl <- temp everywhere (the next
-// X direction's copy of the Picard layer).
+// The step's copies of the state on nodes (i < nx-1, j < ny-1) as k2_copy, with
+// both directions' first copies of the Picard layer: d0..d4 <- src.
 template <class T>
-__global__ void k2_fan(int nx, int ny, L3<T> src, L3<T> d0, L3<T> d1, L3<T> d2, L3<T> d3) {
+__global__ void k2_fan(int nx, int ny, L3<T> src, L3<T> d0, L3<T> d1, L3<T> d2, L3<T> d3, L3<T> d4) {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= (int64_t)nx * ny) return;
     const int i = (int)(q / ny), j = (int)(q % ny);
@@ -89,25 +86,7 @@ __global__ void k2_fan(int nx, int ny, L3<T> src, L3<T> d0, L3<T> d1, L3<T> d2, 
         d1.f[f][q] = v;
         d2.f[f][q] = v;
         d3.f[f][q] = v;
-    }
-}
-
-template <class T>
-__global__ void k2_merge_fan(int nx, int ny, const uint8_t* __restrict__ type, int merge,
-                             L3<T> next, L3<T> temp, L3<T> tl) {
-    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= (int64_t)nx * ny) return;
-    const int i = (int)(q / ny), j = (int)(q % ny);
-    if (i >= nx - 1 || j >= ny - 1) return;
-    const bool in = type[q] == NODE_IN;
-#pragma unroll
-    for (int f = 0; f < 3; f++) {
-        T v = temp.f[f][q];
-        if (in) {
-            v = merge ? (v + next.f[f][q]) / 2 : next.f[f][q];
-            temp.f[f][q] = v;
-        }
-        tl.f[f][q] = v;
+        d4.f[f][q] = v;
     }
 }
 
@@ -129,14 +108,20 @@ __global__ void k2_update_boundaries(int nx, int ny, const uint8_t* __restrict__
     }
 }
 
-// Solver2D::ClearOutterCells (Solver2D.cpp:75-85)
+// End of a step: Solver2D::ClearOutterCells (Solver2D.cpp:75-85) on next, then
+// state <- next (a copy that skips the last row and column).
 template <class T>
-__global__ void k2_clear_outer(int64_t n, const uint8_t* __restrict__ type, L3<T> next, T startT) {
+__global__ void k2_end_step(int nx, int ny, const uint8_t* __restrict__ type, L3<T> next, L3<T> cur, T startT) {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n || type[q] != NODE_OUT) return;
-    next.f[0][q] = 0;
-    next.f[1][q] = 0;
-    next.f[2][q] = startT;
+    if (q >= (int64_t)nx * ny) return;
+    const int i = (int)(q / ny), j = (int)(q % ny);
+    const bool outer = type[q] == NODE_OUT, inner = i < nx - 1 && j < ny - 1;
+#pragma unroll
+    for (int f = 0; f < 3; f++) {
+        const T v = outer ? (f == 2 ? startT : (T)0) : next.f[f][q];
+        if (outer) next.f[f][q] = v;
+        if (inner) cur.f[f][q] = v;
+    }
 }
 
 // Row t of a line system of n rows (BuildMatrix, AdiSolver2D.cpp:118-178, and
@@ -254,8 +239,8 @@ __global__ void k2_sweep(int nsys, const Sys2* __restrict__ sys, int nx, int ny,
 // is eliminated (a thread's global loads would instead queue behind its own
 // scratch stores: one counter covers both on this architecture).
 // mode 0: the solution on every row into `out` (the local result layer);
-// mode 1 (a direction with one inner iteration): the solution into `lt` and
-// `out` on NODE_IN rows off the grid's last row and column, which is what the
+// mode 1 (a direction with one inner iteration): the solution into `lt`, `out`
+// and, where given, `t2` on NODE_IN rows off the grid's last row and column, which is what the
 // direction's copies leave there (SolveDirection, AdiSolver2D.cpp:203-226:
 // the local layer takes the first solve on NODE_IN, the layer and the result
 // are copied out on NODE_IN, both copies skipping the last row and column);
@@ -273,7 +258,7 @@ template <class T, bool DIRX>
 __global__ void __launch_bounds__(kSweepLdsThreads) k2_sweep_lds(
     int nsys, int spw, int nmax, const Sys2* __restrict__ sys, int nx, int ny,
     const uint8_t* __restrict__ type, const uint8_t* __restrict__ bc, L3<T> g, L3<T> lc,
-    L3<T> tl, L3<T> out, L3<T> lt, L3<T> dm, int mode, P2 prm) {
+    L3<T> tl, L3<T> out, L3<T> lt, L3<T> t2, L3<T> dm, int mode, P2 prm) {
     extern __shared__ char smem2[];
     constexpr int R = kSweepBatch;
     const int rs = spw * nmax;  // rows in LDS
@@ -354,12 +339,14 @@ __global__ void __launch_bounds__(kSweepLdsThreads) k2_sweep_lds(
     // (the flag bytes are read in mode 0 too, unused: no load under a branch)
     T* const o1 = out.f[var];
     T* const o2 = mode == 1 ? lt.f[var] : out.f[var];
+    T* const o3 = mode == 1 && t2.f[var] ? t2.f[var] : o2;
     T* const od = dm.f[var];
     auto put = [&](int t, T v, uint8_t f) {
         const int64_t ct = cell(q, t);
         const bool w = mode == 0 || f != 0;
         (w ? o1 : od)[ct] = v;
         (w ? o2 : od)[ct] = v;
+        (w ? o3 : od)[ct] = v;
     };
     T x = dp;
     put(n - 1, x, mf[(n - 1) * spw]);
@@ -444,7 +431,7 @@ template <class T, bool DIRX, int CL>
 __global__ void __launch_bounds__(kSweepLdsThreads) k2_sweep_chunks(
     int nsys, int spw, int nmax, const Sys2* __restrict__ sys, int nx, int ny,
     const uint8_t* __restrict__ type, const uint8_t* __restrict__ bc, L3<T> g, L3<T> lc,
-    L3<T> tl, L3<T> out, L3<T> lt, int mode, P2 prm, int wa, int wb) {
+    L3<T> tl, L3<T> out, L3<T> lt, L3<T> t2, int mode, P2 prm, int wa, int wb) {
     extern __shared__ __align__(16) char smem2[];
     Row4<T>* const rw = reinterpret_cast<Row4<T>*>(smem2);
     const int w = wa + kChunkExact, rows = chunk_rows(nmax, w, wb, CL), pitch = chunk_pitch(rows, CL);
@@ -614,6 +601,7 @@ __global__ void __launch_bounds__(kSweepLdsThreads) k2_sweep_chunks(
     __syncthreads();
     T* const o1 = out.f[var];
     T* const o2 = mode == 1 ? lt.f[var] : o1;
+    T* const o3 = mode == 1 ? t2.f[var] : nullptr;
     for (int e = threadIdx.x; e < spw * nmax; e += blockDim.x) {
         const int sl = DIRX ? e % spw : e / nmax, t = DIRX ? e / spw : e % nmax;
         if (sl >= nloc) continue;
@@ -626,6 +614,7 @@ __global__ void __launch_bounds__(kSweepLdsThreads) k2_sweep_chunks(
             const T v = rw[sl * pitch + u + u / CL].d;
             o1[ct] = v;
             o2[ct] = v;
+            if (o3) o3[ct] = v;
         }
     }
 }
@@ -635,8 +624,8 @@ __global__ void __launch_bounds__(kSweepLdsThreads) k2_sweep_chunks(
 constexpr int kDiv2Blocks = 256;
 
 template <class T>
-__global__ void k2_div(int nx, int ny, const uint8_t* __restrict__ type, L3<T> L, T dx, T dy,
-                       double* __restrict__ part) {
+__device__ __forceinline__ void div_part(int nx, int ny, const uint8_t* __restrict__ type, const L3<T>& L,
+                                         T dx, T dy, double* __restrict__ part) {
     __shared__ double ssum[kBS2], scnt[kBS2];
     double sum = 0, cnt = 0;
     const int64_t n = (int64_t)(nx - 1) * (ny - 1);
@@ -671,12 +660,47 @@ __global__ void k2_div(int nx, int ny, const uint8_t* __restrict__ type, L3<T> L
     }
 }
 
-// One work-group of kDiv2Blocks threads: the partials come into LDS in one
-// parallel load, then thread 0 adds them in block order.
+template <class T>
+__global__ void k2_div(int nx, int ny, const uint8_t* __restrict__ type, L3<T> L, T dx, T dy,
+                       double* __restrict__ part) {
+    div_part<T>(nx, ny, type, L, dx, dy, part);
+}
+
+// End of a Picard iteration of the one-iteration path: temp <- next on NODE_IN
+// (merge: (temp + next) / 2), tl and tl2 <- temp everywhere (both directions'
+// next copies of the Picard layer), on nodes (i < nx-1, j < ny-1) as k2_copy, and
+// the partial sums of next's divergence error.  Apart, with the copy before the Y
+// direction, these were four launches of about 4.5 us each.
+template <class T>
+__global__ void __launch_bounds__(kBS2) k2_merge_div(int nx, int ny, const uint8_t* __restrict__ type,
+                                                     int merge, L3<T> next, L3<T> temp, L3<T> tl, L3<T> tl2,
+                                                     T dx, T dy, double* __restrict__ part) {
+    const int64_t n = (int64_t)nx * ny;
+    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n;
+         q += (int64_t)gridDim.x * blockDim.x) {
+        const int i = (int)(q / ny), j = (int)(q % ny);
+        if (i >= nx - 1 || j >= ny - 1) continue;
+        const bool in = type[q] == NODE_IN;
+#pragma unroll
+        for (int f = 0; f < 3; f++) {
+            T v = temp.f[f][q];
+            if (in) {
+                v = merge ? (v + next.f[f][q]) / 2 : next.f[f][q];
+                temp.f[f][q] = v;
+            }
+            tl.f[f][q] = v;
+            tl2.f[f][q] = v;
+        }
+    }
+    div_part<T>(nx, ny, type, next, dx, dy, part);
+}
+
+// One work-group of kDiv2Blocks threads per slot: its partials come into LDS in
+// one parallel load, then thread 0 adds them in block order.
 __global__ void __launch_bounds__(kDiv2Blocks) k2_div_finish(const double* __restrict__ part,
                                                              int nb, double* __restrict__ out) {
     __shared__ double sp[2 * kDiv2Blocks];
-    for (int k = threadIdx.x; k < 2 * nb; k += blockDim.x) sp[k] = part[k];
+    for (int k = threadIdx.x; k < 2 * nb; k += blockDim.x) sp[k] = part[(int64_t)blockIdx.x * 2 * nb + k];
     __syncthreads();
     if (threadIdx.x != 0) return;
     double s = 0, c = 0;
@@ -684,8 +708,8 @@ __global__ void __launch_bounds__(kDiv2Blocks) k2_div_finish(const double* __res
         s += sp[2 * b];
         c += sp[2 * b + 1];
     }
-    out[0] = s;
-    out[1] = c;
+    out[2 * blockIdx.x] = s;
+    out[2 * blockIdx.x + 1] = c;
 }
 
 
@@ -1407,8 +1431,8 @@ class Solver2D final : public ISolver2 {
     P2 prm{};
     double startT;
     uint8_t *d_type = nullptr, *d_bc = nullptr;
-    T* buf = nullptr;  // 7 layers x 3 fields: g, cur, next, half, temp, tl, nl
-    L3<T> g{}, cur{}, next{}, half{}, temp{}, tl{}, nl{};
+    T* buf = nullptr;  // 8 layers x 3 fields: g, cur, next, half, temp, tl, nl, tl2
+    L3<T> g{}, cur{}, next{}, half{}, temp{}, tl{}, nl{}, tl2{};
     Sys2 *d_rows = nullptr, *d_cols = nullptr;
     int nrows = 0, ncols = 0;
     int rows_nmax = 0, cols_nmax = 0;  // longest system of each direction
@@ -1450,10 +1474,10 @@ class Solver2D final : public ISolver2 {
         startT = d->start_t;
         CMCX_HIP(hipMalloc((void**)&d_type, N));
         CMCX_HIP(hipMalloc((void**)&d_bc, N));
-        CMCX_HIP(hipMalloc((void**)&buf, sizeof(T) * N * 21));
-        CMCX_HIP(hipMemsetAsync(buf, 0, sizeof(T) * N * 21, st));
-        L3<T>* Ls[7] = {&g, &cur, &next, &half, &temp, &tl, &nl};
-        for (int l = 0; l < 7; l++)
+        CMCX_HIP(hipMalloc((void**)&buf, sizeof(T) * N * 24));
+        CMCX_HIP(hipMemsetAsync(buf, 0, sizeof(T) * N * 24, st));
+        L3<T>* Ls[8] = {&g, &cur, &next, &half, &temp, &tl, &nl, &tl2};
+        for (int l = 0; l < 8; l++)
             for (int f = 0; f < 3; f++) Ls[l]->f[f] = buf + (int64_t)(l * 3 + f) * N;
         CMCX_HIP(hipMemcpyAsync(d_type, d->type, N, hipMemcpyHostToDevice, st));
         CMCX_HIP(hipMemcpyAsync(d_bc, d->bc, N, hipMemcpyHostToDevice, st));
@@ -1470,7 +1494,7 @@ class Solver2D final : public ISolver2 {
         }
         if (method == CMCX2D_STABLE) build_relaxation(d->type);
         else build_systems(d->type);
-        CMCX_HIP(hipMalloc((void**)&d_part, sizeof(double) * 2 * kDiv2Blocks));
+        CMCX_HIP(hipMalloc((void**)&d_part, sizeof(double) * 2 * kDiv2Blocks * kErrSlots));
         CMCX_HIP(hipMalloc((void**)&d_err, sizeof(double) * 2 * kErrSlots));
         CMCX_HIP(hipHostMalloc((void**)&h_err, sizeof(double) * 2 * kErrSlots, hipHostMallocDefault));
         if (method == CMCX2D_STABLE) {
@@ -1768,7 +1792,7 @@ class Solver2D final : public ISolver2 {
 
     // mode 1: k2_sweep_lds writes lt and out on the NODE_IN rows (a direction
     // with one inner iteration), else the solution into out
-    void sweep_lds(bool dirx, int spw, int mode, L3<T> lc, L3<T> tlc, L3<T> out, L3<T> lt) {
+    void sweep_lds(bool dirx, int spw, int mode, L3<T> lc, L3<T> tlc, L3<T> out, L3<T> lt, L3<T> t2 = {}) {
         const int n = dirx ? nrows : ncols, nmax = dirx ? rows_nmax : cols_nmax;
         if (const int early = early_rows(dirx)) {
             // a wavefront per system
@@ -1781,7 +1805,7 @@ class Solver2D final : public ISolver2 {
                              : (cl == 4 ? k2_sweep_chunks<T, false, 4> : k2_sweep_chunks<T, false, 8>);
             hipLaunchKernelGGL(kern, dim3((unsigned)((n + per - 1) / per), 3), dim3(kSweepLdsThreads),
                                (size_t)per * pitch * sizeof(Row4<T>), st, n, per, nmax, dirx ? d_rows : d_cols, nx, ny, d_type,
-                               d_bc, g, lc, tlc, out, lt, mode, prm, wa, wb);
+                               d_bc, g, lc, tlc, out, lt, t2, mode, prm, wa, wb);
             CMCX_LAUNCH_CHECK();
             return;
         }
@@ -1789,11 +1813,11 @@ class Solver2D final : public ISolver2 {
         const dim3 grid((unsigned)((n + spw - 1) / spw), 3);
         if (dirx)
             hipLaunchKernelGGL((k2_sweep_lds<T, true>), grid, dim3(kSweepLdsThreads), lds, st, n,
-                               spw, nmax, d_rows, nx, ny, d_type, d_bc, g, lc, tlc, out, lt, nl,
+                               spw, nmax, d_rows, nx, ny, d_type, d_bc, g, lc, tlc, out, lt, t2, nl,
                                mode, prm);
         else
             hipLaunchKernelGGL((k2_sweep_lds<T, false>), grid, dim3(kSweepLdsThreads), lds, st, n,
-                               spw, nmax, d_cols, nx, ny, d_type, d_bc, g, lc, tlc, out, lt, nl,
+                               spw, nmax, d_cols, nx, ny, d_type, d_bc, g, lc, tlc, out, lt, t2, nl,
                                mode, prm);
         CMCX_LAUNCH_CHECK();
     }
@@ -1817,10 +1841,10 @@ class Solver2D final : public ISolver2 {
         CMCX_LAUNCH_CHECK();
     }
 
-    // AdiSolver2D::SolveDirection; tl_ready: tl already holds lt (a fused copy)
-    void direction(bool dirx, int L, L3<T> lc, L3<T> lt, L3<T> out, bool tl_ready = false) {
+    // AdiSolver2D::SolveDirection
+    void direction(bool dirx, int L, L3<T> lc, L3<T> lt, L3<T> out) {
         if (!(dirx ? nrows : ncols)) return;  // the reference reads list[0] unconditionally
-        if (!tl_ready) copy(lt, tl, kAll, 0);
+        copy(lt, tl, kAll, 0);
         if (L == 1) {
             if (const int spw = lds_spw(dirx)) {
                 // the solve writes what the copies below would leave on NODE_IN
@@ -1857,6 +1881,12 @@ class Solver2D final : public ISolver2 {
         div_enqueue(Lr, 0);
         read_errors(1);
         return h_err[0] / h_err[1];
+    }
+
+    void end_step() {
+        hipLaunchKernelGGL((k2_end_step<T>), dim3(blocks2(N)), dim3(kBS2), 0, st, nx, ny, d_type, next, cur,
+                           (T)startT);
+        CMCX_LAUNCH_CHECK();
     }
 
     int update_boundaries() override {
@@ -1963,10 +1993,7 @@ class Solver2D final : public ISolver2 {
                 return CMCX_ERR_PICARD;
             }
         }
-        hipLaunchKernelGGL((k2_clear_outer<T>), dim3(blocks2(N)), dim3(kBS2), 0, st, N, d_type, next,
-                           (T)startT);
-        CMCX_LAUNCH_CHECK();
-        copy(next, cur, kAll, 0);
+        end_step();
         CMCX_HIP(hipStreamSynchronize(st));
         if (err_out) *err_out = err;
         if (iters) *iters = it;
@@ -1981,14 +2008,13 @@ class Solver2D final : public ISolver2 {
         const bool fused = one_pass(L);
         if (fused) {
             hipLaunchKernelGGL((k2_fan<T>), dim3(blocks2(N)), dim3(kBS2), 0, st, nx, ny, cur, next,
-                               half, temp, tl);
+                               half, temp, tl, tl2);
             CMCX_LAUNCH_CHECK();
         } else {
             copy(cur, next, kAll, 0);
             copy(cur, half, kAll, 0);
             copy(cur, temp, kAll, 0);
         }
-        bool tl_ready = fused;  // tl holds temp (k2_fan, k2_merge_fan)
         // the error before the loop decides only whether a step with G = 0 iterates
         double err = G == 0 ? div_error(next) : 0.0;
         int it = 0;
@@ -1999,18 +2025,25 @@ class Solver2D final : public ISolver2 {
         // which the next step's copies overwrite before anything reads them.
         const int batch = std::min(G, (int)kErrSlots);
         for (int k = 0; k < batch; k++) {
-            direction(true, L, cur, temp, half, tl_ready);
-            direction(false, L, half, temp, next);
-            div_enqueue(next, k);
-            if (fused && k + 1 < batch) {
-                hipLaunchKernelGGL((k2_merge_fan<T>), dim3(blocks2(N)), dim3(kBS2), 0, st, nx, ny,
-                                   d_type, k == 0 ? 0 : 1, next, temp, tl);
+            if (fused) {
+                // tl and tl2 hold the Picard layer (k2_fan, k2_merge_div); the X
+                // sweep keeps tl2 up to date for the Y sweep
+                sweep_lds(true, lds_spw(true), 1, cur, tl, half, temp, tl2);
+                sweep_lds(false, lds_spw(false), 1, half, tl2, next, temp);
+                hipLaunchKernelGGL((k2_merge_div<T>), dim3(kDiv2Blocks), dim3(kBS2), 0, st, nx, ny, d_type,
+                                   k == 0 ? 0 : 1, next, temp, tl, tl2, (T)prm.dx, (T)prm.dy,
+                                   d_part + (int64_t)k * 2 * kDiv2Blocks);
                 CMCX_LAUNCH_CHECK();
-                tl_ready = true;
             } else {
+                direction(true, L, cur, temp, half);
+                direction(false, L, half, temp, next);
+                div_enqueue(next, k);
                 copy(next, temp, kIn, k == 0 ? 0 : 1);
-                tl_ready = false;
             }
+        }
+        if (fused && batch > 0) {
+            hipLaunchKernelGGL(k2_div_finish, dim3(batch), dim3(kDiv2Blocks), 0, st, d_part, kDiv2Blocks, d_err);
+            CMCX_LAUNCH_CHECK();
         }
         if (batch > 0) {
             read_errors(batch);
@@ -2039,10 +2072,7 @@ class Solver2D final : public ISolver2 {
                 return CMCX_ERR_PICARD;
             }
         }
-        hipLaunchKernelGGL((k2_clear_outer<T>), dim3(blocks2(N)), dim3(kBS2), 0, st, N, d_type,
-                           next, (T)startT);
-        CMCX_LAUNCH_CHECK();
-        copy(next, cur, kAll, 0);
+        end_step();
         CMCX_HIP(hipStreamSynchronize(st));
         if (err_out) *err_out = err;
         if (iters) *iters = it;
