@@ -865,7 +865,9 @@ bool fused_variant_ok(int n, int v) {
 // / 402); shorter ones lose (64^3 +5 %).
 // X and Y: up to 64 tiles of 128-byte rows leave most of the 256 CUs idle, so
 // lines of at most 64 nodes take 32-byte tiles of 4-row chunks (24^3 and 32^3:
-// FP32 step 80 / 73 us, FP64 101 / 92).  Otherwise 128-byte tiles; the Picard
+// FP32 step 80 / 73 us, FP64 101 / 92), longer ones 32-byte tiles of 8-row chunks
+// up to 80 and 64-byte tiles up to 128 (FP32 189 x 39 x 40, 78 X tiles: 164 / 152
+// us; FP64 35 x 158 x 33, 105 Y tiles: 194 / 177).  Otherwise 128-byte tiles; the Picard
 // layer is parked in LDS for the merge once its four fields are 8 MiB, a quarter
 // of the chip's L2: the second read of a smaller one hits there (64^3 FP32: 112 us
 // read again, 115 parked), that of a larger one goes further out (FP32 128^3
@@ -885,6 +887,7 @@ int fused_default_variant(const std::vector<Geom>& gs, int axis) {
         return sizeof(T) == 8 && n >= 96 ? 7 : 0;
     }
     if (n <= 64 && tiles <= 64) return 5;
+    if (tiles <= 128) return tiles <= 80 ? 2 : 1;
     return bytes >= (8 << 20) && strided_variant_fits<T>(n, 6) ? 6 : 0;
 }
 

@@ -13,7 +13,7 @@ from gpu_util import rel_l2_scaled, say, vel_norm
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(32, 32, 32), (64, 21, 33), (65, 32, 32), (40, 40, 40), (86, 75, 82), (12, 9, 95), (12, 9, 96),
-          (12, 9, 128), (12, 9, 129), (256, 40, 64)]
+          (12, 9, 128), (12, 9, 129), (256, 40, 64), (90, 25, 40), (189, 60, 20), (130, 129, 8)]
 
 
 def _same(a, b, dtype):
