@@ -176,6 +176,7 @@ class Solver final : public ISolver {
         T* tape = nullptr;     // per step: S, Picard layers 1..3G, sweep outputs 0..3G-1
         int64_t tape_layers = 0;
         int tape_G = 0;
+        bool tape_values = false;  // the Picard-layer slots hold the node values
         int nbuf = 0;              // tape buffers (two when the rollout has several intervals)
         int holds[2] = {-1, -1};   // interval each tape buffer holds (-1 = none)
         hipStream_t fs = nullptr;  // stream of the recompute, beside the reverse on `st`
@@ -954,6 +955,7 @@ class Solver final : public ISolver {
                 return CMCX_ERR_ARG;
             }
         invalidate_recording("set_boundary");
+        adj.tape_values = false;
         std::memcpy(&h_bcv[o], bv, N);
         std::memcpy(&h_bct[o], bt, N);
         CMCX_HIP(hipMemcpyAsync(d_bcv + o, bv, N, hipMemcpyHostToDevice, st));
@@ -1180,7 +1182,7 @@ class Solver final : public ISolver {
         adj.G = G;
         adj.steps = steps;
         adj.every = every;
-        ensure_tape(true);
+        ensure_tape();
         // the last intervals, one per tape buffer, are recorded on the way
         // (their layers go to the tape instead of the step buffers), so the
         // backward pass recomputes only the intervals before them, and starts
@@ -1217,8 +1219,9 @@ class Solver final : public ISolver {
     // than one interval (the backward pass recomputes one interval while it
     // reverses the next), else one.  The Picard-layer slots hold the node
     // values on non-IN nodes (the forward's temp holds the boundary-filled state
-    // there, and the sweeps write NODE_IN nodes only).
-    void ensure_tape(bool init_slots) {
+    // there, and the sweeps write NODE_IN nodes only), put there when the tape
+    // is allocated and again after new node values.
+    void ensure_tape() {
         const int64_t per = 1 + 6 * (int64_t)adj.G;
         const int64_t nsteps_tape = std::min(adj.every, adj.steps);
         const int nbuf = adj.steps > adj.every ? 2 : 1;
@@ -1229,19 +1232,15 @@ class Solver final : public ISolver {
             CMCX_HIP(hipMalloc((void**)&adj.tape, sizeof(T) * (4 * NT * need + kSlack)));
             adj.tape_layers = need;
             adj.tape_G = adj.G;
+            adj.tape_values = false;
             adj.holds[0] = adj.holds[1] = -1;
-            init_slots = true;
         }
         adj.nbuf = nbuf;
-        if (init_slots) {  // node values may have changed since the last recording
+        if (!adj.tape_values) {
             Layer4<T> gl;
             for (int f = 0; f < 4; f++) gl.f[f] = d_g[f];
-            for (int64_t i = 0; i < adj.tape_layers / per; i++)
-                for (int k = 1; k <= 3 * adj.G; k += 2) {
-                    Layer4<T> a = lay(adj.tape + i * per * 4 * NT, k);
-                    Layer4<T> b = k + 1 <= 3 * adj.G ? lay(adj.tape + i * per * 4 * NT, k + 1) : a;
-                    launch_prep_step_list<T>(n_nonin, d_nonin, d_type, gl, a, a, b, st);
-                }
+            launch_tape_values<T>(n_nonin, d_nonin, gl, adj.tape, NT, per, 3 * adj.G, adj.tape_layers / per, st);
+            adj.tape_values = true;
         }
     }
 
@@ -1309,7 +1308,7 @@ class Solver final : public ISolver {
         }
         const Geom& g = grids[0].g;
         const int64_t per = 1 + 6 * (int64_t)adj.G;
-        ensure_tape(false);
+        ensure_tape();
         if (!adj.work) {
             CMCX_HIP(hipMalloc((void**)&adj.work, sizeof(T) * (4 * NT * 6 + kSlack)));
             CMCX_HIP(hipMalloc((void**)&adj.pp, sizeof(double) * 4 * adj_point_blocks()));

@@ -202,6 +202,11 @@ void launch_adj_sweep(const Geom& g, int axis, const SweepParams<T>& p, const ui
 // neighbours), built once per backward pass: N 16-bit words.
 void launch_adj_mask(const Geom& g, const uint8_t* type, const uint8_t* bcv, const uint8_t* bct,
                      uint16_t* mask, hipStream_t st);
+// Node values g on the listed nodes of layers 1 .. layers of every step's slot of
+// a tape (`per` layers of 4 fields of `pitch` elements per step), one launch.
+template <class T>
+void launch_tape_values(int64_t n, const uint32_t* ids, Layer4<T> g, T* tape, int64_t pitch, int64_t per,
+                        int layers, int64_t steps, hipStream_t st);
 // dst <- src, four fields of n elements, one launch.
 template <class T>
 void launch_copy4(Layer4<T> dst, Layer4<T> src, int64_t n, hipStream_t st);

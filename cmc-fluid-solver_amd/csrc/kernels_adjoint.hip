@@ -431,14 +431,10 @@ __global__ void __launch_bounds__(256) adj_point_kernel(Geom g, SweepParams<T> p
             return (uint32_t)((int)q + (off & -(int)in));
         };
         const int mq = nmask[q];  // node type, BC kinds, NODE_IN neighbours
-        // node-value gradient and state-adjoint accumulator, read whatever the
-        // node types (their updates below are conditional)
-        T gbq[4], caq[4];
+        // state-adjoint accumulator, read whatever the node type
+        T caq[4];
 #pragma unroll
-        for (int f = 0; f < 4; f++) {
-            gbq[f] = gb.f[f][q];
-            caq[f] = last ? cacc.f[f][q] : (T)0;
-        }
+        for (int f = 0; f < 4; f++) caq[f] = last ? cacc.f[f][q] : (T)0;
 
         // own row: lam, the sweep output around q, the T and velocity stencils
         T tbq[4], l[4], xm[4], x0[4], xp[4];
@@ -478,15 +474,34 @@ __global__ void __launch_bounds__(256) adj_point_kernel(Geom g, SweepParams<T> p
                 ra[nb][o] = (F[o][at(o, k, A, 1)] - F[o][at(o, k, A, -1)]) * ia;
             }
         }
+        // the node word, which was asked for first, says which nodes need the
+        // node-value gradient: its loads join those above, which are in flight
+        // (reading it on every node was 4 of some 24 fields per sweep)
+        asm volatile("" ::"v"(mq));
+        const int tq = mq & 3;
+        const bool inq = tq == NODE_IN;
+        // the rows either side: NODE_IN or not (kOutside stands for any other)
+        uint8_t tn[6];
+#pragma unroll
+        for (int nb = 0; nb < 6; nb++) tn[nb] = (mq >> (kMaskNb + nb)) & 1 ? (uint8_t)NODE_IN : kOutside;
+        const bool doxg = last && (tq == NODE_BOUND || tq == NODE_VALVE);
+        const int rl = row_role((uint8_t)tq, tn[2 * A], tn[2 * A + 1]);
+        const bool bnd = rl != RL_IN && rl != RL_NONE;
+        const bool ends = rl == RL_START || rl == RL_END;
+        const bool gv = bnd && (!ends || !(mq & kMaskFreeV)), gt = bnd && (!ends || !(mq & kMaskFreeT));
+        T gbq[4] = {0, 0, 0, 0};
+        if (gv || gt || doxg) {
+#pragma unroll
+            for (int f = 0; f < 4; f++) gbq[f] = gb.f[f][q];
+        }
         // every value above is used here, once, all together: a value used
         // under a condition only would be loaded there, behind its own wait
-        asm volatile("" ::"v"(mq));
 #pragma unroll
         for (int nb = 0; nb < 6; nb++) asm volatile("" ::"v"(kr[nb]));
 #pragma unroll
         for (int f = 0; f < 4; f++)
             asm volatile("" ::"v"(tbq[f]), "v"(l[f]), "v"(xm[f]), "v"(x0[f]), "v"(xp[f]),
-                         "v"(gbq[f]), "v"(caq[f]));
+                         "v"(caq[f]));
         asm volatile("" ::"v"(tgrad));
 #pragma unroll
         for (int f = 0; f < 3; f++) asm volatile("" ::"v"(da[f]));
@@ -507,14 +522,6 @@ __global__ void __launch_bounds__(256) adj_point_kernel(Geom g, SweepParams<T> p
                 asm volatile("" ::"v"(ra[nb][o]));
             }
         }
-        const int tq = mq & 3;
-        const bool inq = tq == NODE_IN;
-        // the rows either side: NODE_IN or not (kOutside stands for any other)
-        uint8_t tn[6];
-#pragma unroll
-        for (int nb = 0; nb < 6; nb++) tn[nb] = (mq >> (kMaskNb + nb)) & 1 ? (uint8_t)NODE_IN : kOutside;
-        const bool doxg = last && (tq == NODE_BOUND || tq == NODE_VALVE);
-
         T acc[4];
 #pragma unroll
         for (int f = 0; f < 4; f++) acc[f] = inq ? alpha * tbq[f] : tbq[f];
@@ -559,10 +566,6 @@ __global__ void __launch_bounds__(256) adj_point_kernel(Geom g, SweepParams<T> p
         // node-value gradient: lam on the sweep's boundary rows whose RHS is the
         // node value (both matrices separately), and at the end of a reversed
         // step tbar on BOUND/VALVE nodes
-        const int rl = row_role((uint8_t)tq, tn[2 * A], tn[2 * A + 1]);
-        const bool bnd = rl != RL_IN && rl != RL_NONE;
-        const bool ends = rl == RL_START || rl == RL_END;
-        const bool gv = bnd && (!ends || !(mq & kMaskFreeV)), gt = bnd && (!ends || !(mq & kMaskFreeT));
 #pragma unroll
         for (int f = 0; f < 4; f++) {
             const bool gl = f < 3 ? gv : gt;
