@@ -118,6 +118,7 @@ struct FusedWork {
     int32_t* d_inst = nullptr;   // Z: grid of each work-group
     int maxn = 0;                // longest line along the axis over the grids
     int kmax = 1;                // X/Y: tiles per work item
+    int one = 0;                 // the launch covers one grid
     int stream = 0;              // sweeps store past the caches (kStoreStream)
     void release();
 };

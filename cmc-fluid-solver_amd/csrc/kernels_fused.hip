@@ -445,7 +445,7 @@ __device__ __forceinline__ void strided_tile(const InstDesc<T>* __restrict__ ins
                                              const Layer4<T>& in, const Layer4<T>& tin,
                                              const Layer4<T>& out, const Layer4<T>& tout,
                                              int merges, int stores,
-                                             const int32_t* __restrict__ work, int kmax) {
+                                             const int32_t* __restrict__ work, int kmax, int one) {
     extern __shared__ char smem_raw[];
     T* red = reinterpret_cast<T*>(smem_raw);
     constexpr int GPW = 64 / LPG;  // chunks (lane groups) per wave
@@ -456,16 +456,24 @@ __device__ __forceinline__ void strided_tile(const InstDesc<T>* __restrict__ ins
     const int chunk = wave * GPW + lane / LPG;
     const int P = nw * GPW;
 
-    // work item: the instance and up to kmax of its tiles (tile = outer *
-    // ztiles + z tile, -1 = none).  The work-group is sized for the longest
+    // work item: the instance and up to kmax of its tiles (outer index << 8 |
+    // z tile, -1 = none).  The work-group is sized for the longest
     // line of the batch; a grid with shorter lines packs several tiles into
     // it, tile k on chunks [k * cpl, (k + 1) * cpl) of each z-line slot.  The
     // lines laid end to end form one block-diagonal system (a line starts and
     // ends on a non-IN face node, whose row does not reach across), so the
-    // reduced solve treats them as one line.
+    // reduced solve treats them as one line.  With one grid (`one`) its
+    // descriptor is read beside the item, not after it, and with one tile per
+    // item no division finds the tile: on small grids the kernel is little more
+    // than this chain of loads and the one that follows (64^3 FP32 X 7.9 -> 7.6,
+    // Y 9.7 -> 9.5 us; the Z sweep gains nothing from it).
     const int b = (int)xcd_remap(blockIdx.x, gridDim.x);
     const int32_t* item = work + (int64_t)b * (kmax + 1);
-    const int inst = item[0];
+    int inst = 0;
+    if (!one) {
+        inst = item[0];
+        asm volatile("" : "+s"(inst));  // (a branch, not a select that waits for the item)
+    }
     const Geom g = insts[inst].g;
     SweepParams<T> p = insts[inst].p[AXIS];
     p.three_dt = three_dt;
@@ -473,11 +481,16 @@ __device__ __forceinline__ void strided_tile(const InstDesc<T>* __restrict__ ins
     const int n = AXIS == AX_X ? g.nx : g.ny;
     const int s = AXIS == AX_X ? (int)g.sx : (int)g.sy;
     const int cpl = (n + M - 1) / M;  // chunks per line of this grid
-    const int k = chunk / cpl;
-    const int tile = k < kmax ? item[1 + k] : -1;
-    const int ztiles = (g.nz + LPG - 1) / LPG;
-    const int outer = tile >= 0 ? tile / ztiles : 0;
-    const int z = (tile >= 0 ? tile % ztiles : 0) * LPG + gl;
+    int k = 0, tile;
+    if (kmax == 1) {
+        tile = item[1];
+        if (chunk >= cpl) tile = -1;
+    } else {
+        k = chunk / cpl;
+        tile = k < kmax ? item[1 + k] : -1;
+    }
+    const int outer = tile >= 0 ? tile >> 8 : 0;
+    const int z = (tile >= 0 ? tile & 255 : 0) * LPG + gl;
     const bool zok = tile >= 0 && z < g.nz;
     // the grid's own arrays, and its rows as byte offsets in them (lines of a
     // tile have x, y in [1, n-2] across the sweep: their neighbour lines exist)
@@ -533,10 +546,10 @@ __global__ void __launch_bounds__(MAXT, MINW) fused_strided_kernel(
     const InstDesc<T>* __restrict__ insts, T three_dt, const uint8_t* __restrict__ type,
     const T* __restrict__ gv0, const T* __restrict__ gv1, const T* __restrict__ gv2,
     const T* __restrict__ gv3, Layer4<T> in, Layer4<T> tin, Layer4<T> out, Layer4<T> tout,
-    int merges, int stores, const int32_t* __restrict__ work, int kmax) {
+    int merges, int stores, const int32_t* __restrict__ work, int kmax, int one) {
     const T* gval[4] = {gv0, gv1, gv2, gv3};
     strided_tile<T, AXIS, M, LPG, KEEP, BSYNC>(insts, three_dt, type, gval, in, tin, out, tout,
-                                               merges, stores, work, kmax);
+                                               merges, stores, work, kmax, one);
 }
 
 // Contiguous lines (Z sweep): 32 lanes per line, two lines per wavefront.  A
@@ -955,7 +968,7 @@ void launch_fused_sweep(const InstDesc<T>* insts, T three_dt, int axis, const Fu
                                              16 / (int)sizeof(T), kShapes[V].keep, BS>),          \
                        dim3(blocks), dim3(64 * waves), lds, st, insts, three_dt, tflags, gval[0], \
                        gval[1], gval[2], gval[3], in, tin, out, tout, merges, stores, w.d_items, \
-                       w.kmax)
+                       w.kmax, w.one)
 #define LSA(AX)                                 \
     if (bsync) {                                \
         switch (variant) {                      \
@@ -1011,9 +1024,9 @@ void FusedWork::release() {
 //      (capacity = 32 lanes x the rows per lane of the longest line), each
 //      instance's slots padded with (-1, 0) to whole work-groups (2 per wave),
 //      plus the instance of every work-group.
-//   X/Y: items of kmax + 1 ints: (instance, tile, tile, ...), tile = outer *
-//      ztiles + z tile of the tiles of lpg z lines holding a NODE_IN node,
-//      -1-padded; an instance takes floor(P / chunks per line) tiles per item
+//   X/Y: items of kmax + 1 ints: (instance, tile, tile, ...), tile = outer <<
+//      8 | z tile of the tiles of lpg z lines holding a NODE_IN node (z lines of
+//      at most 512 nodes, at least 4 to a tile), -1-padded; an instance takes floor(P / chunks per line) tiles per item
 //      (P = chunks per z-line slot of the work-group, chunks of m rows).
 void build_fused_work(const uint8_t* h_type, const std::vector<Geom>& geoms,
                       const std::vector<int64_t>& offs, int axis, int lpg, int m, size_t elem,
@@ -1034,6 +1047,7 @@ void build_fused_work(const uint8_t* h_type, const std::vector<Geom>& geoms,
     }
     w.maxn = 0;
     w.kmax = 1;
+    w.one = geoms.size() == 1;
     for (const Geom& g : geoms)
         w.maxn = std::max(w.maxn, axis == AX_Z ? g.nz : axis == AX_X ? g.nx : g.ny);
     if (axis == AX_Z) {
@@ -1093,7 +1107,7 @@ void build_fused_work(const uint8_t* h_type, const std::vector<Geom>& geoms,
                     for (int r = 0; r < n && !any; r++)
                         for (int z = zt * lpg; z < std::min(g.nz, (zt + 1) * lpg) && !any; z++)
                             any = t[o * so + r * sr + z] == NODE_IN;
-                    if (any) tiles[i].push_back(o * ztiles + zt);
+                    if (any) tiles[i].push_back(o << 8 | zt);
                 }
         }
         const int W = w.kmax + 1;
