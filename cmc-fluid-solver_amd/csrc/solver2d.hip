@@ -1083,8 +1083,8 @@ __global__ void __launch_bounds__(1024) k2s_poisson(
 //     ahead; kNotInner marks the other cells, so that no flags are read.
 //   * the stopping test works on lane masks, in scalar registers: per sweep and
 //     row a NaN, and a change of tol or more since the row's last NaN.
-// Per sweep of a 120 x 135 grid in FP64: 39.6 us before, 7.0 now; with one sweep
-// per lane 8.2, with four 8.6 (scalar registers spill).  A first form with rows
+// Per sweep of a 120 x 135 grid in FP64: 39.6 us before, 6.7 now; with one sweep
+// per lane a sixth more, with four a fifth (scalar registers spill).  A first form with rows
 // of q in LDS, where a lane moves on to its next sweep by itself in a branch
 // that some lane takes on every step, took 7.7 to 8.6.
 constexpr int kPoisGroup = 256;              // sweeps of a group at most
@@ -1154,7 +1154,7 @@ __global__ void __launch_bounds__(1024) k2s_poisson_lds(
             // Branch-free but for the rare cases (a change too close to tol to
             // tell, the end of a turn), each tested once for the MW cells.
             const int w0 = __builtin_amdgcn_readfirstlane(r);  // the wavefront's first row
-            const int late = w0 / P, wr = w0 - late * P;       // its delay in turns, its first row's residue at x = 0
+            const int late = __builtin_amdgcn_readfirstlane(w0 / P), wr = w0 - late * P;       // its delay in turns, its first row's residue at x = 0
             const uint64_t rows = nx - w0 >= 64 ? ~0ull : nx > w0 ? (1ull << (nx - w0)) - 1 : 0;
             const uint32_t qb = (uint32_t)Q * (uint32_t)sizeof(T), pb = (uint32_t)P * qb;  // bytes of a row, of q
             // lanes beyond the rows read the last one's cells and are never live
@@ -1174,15 +1174,12 @@ __global__ void __launch_bounds__(1024) k2s_poisson_lds(
             };
             // dvs two steps on, its row's residue the first member's
             const uint32_t db = (uint32_t)rp * (uint32_t)sizeof(double);
-            int res2 = __builtin_amdgcn_readfirstlane((P - (k0 + 2) % P) % P);
-            const char* drow = reinterpret_cast<const char*>(dvs) + (int64_t)res2 * db;
-            auto advance_dvs = [&] {
-                res2++;
-                drow += db;
-                if (res2 == P) {
-                    res2 = 0;
-                    drow = reinterpret_cast<const char*>(dvs);
-                }
+            const int res2 = __builtin_amdgcn_readfirstlane((P - (k0 + 2) % P) % P);
+            uint32_t drow = (uint32_t)res2 * db;
+            const uint32_t dend = (uint32_t)P * db;
+            auto advance_dvs = [&] { drow = drow + db == dend ? 0 : drow + db; };
+            auto dvs_at = [&](int u) {
+                return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(dvs) + (voff[u] + drow));
             };
 #pragma unroll
             for (int u = 0; u < MW; u++) {
@@ -1202,7 +1199,7 @@ __global__ void __launch_bounds__(1024) k2s_poisson_lds(
 #pragma unroll
             for (int h = 0; h < 2; h++) {
 #pragma unroll
-                for (int u = 0; u < MW; u++) dv[u][h] = *reinterpret_cast<const double*>(drow + voff[u]);
+                for (int u = 0; u < MW; u++) dv[u][h] = dvs_at(u);
                 advance_dvs();
             }
             // (waited for here: loads outstanding at the loop's entry would make
@@ -1277,8 +1274,10 @@ __global__ void __launch_bounds__(1024) k2s_poisson_lds(
                             res[u] = 0;
                             newest[u] = 0;
                         }
-                        newest[u] = newest[u] << 1 | (uint64_t)(res[u] >= wr);
-                        dv[u][h] = *reinterpret_cast<const double*>(drow + voff[u]);
+                        // (res >= wr as bit arithmetic: a comparison's result would go
+                        // through the vector unit)
+                        newest[u] = newest[u] << 1 | (uint64_t)((uint32_t)~(res[u] - wr) >> 31);
+                        dv[u][h] = dvs_at(u);
                     }
                     advance_dvs();
                     step_barrier();
