@@ -44,9 +44,11 @@
 // (at_byte), the stores' switches are outside the row loops, and the dissipation
 // takes its differences from the advection term.  With the rows handled one by
 // one, selects for every role and a 64-bit address per access (over 300 per
-// row) the sweeps took, X / Y / Z in us: 32^3 FP32 9.3 / 9.9 / 5.0, now 6.6 /
-// 7.5 / 3.8; 64^3 11.2 / 12.3 / 9.2, now 8.3 / 10.5 / 7.6; 250 x 203 x 187 167
-// / 202 / 142, now 152 / 190 / 142; 256^3 267 / 303 / 187, now 261 / 272 / 185.
+// row) the sweeps took, on 128-byte tiles, X / Y / Z in us: 32^3 FP32 9.3 / 9.9 /
+// 5.0, so 6.6 / 7.5 / 3.8; 64^3 11.2 / 12.3 / 9.2, so 8.3 / 10.5 / 7.6; 250 x 203
+// x 187 167 / 202 / 142, so 152 / 190 / 142; 256^3 267 / 303 / 187, so 261 / 272
+// / 185.  (Tiles chosen by size, fused_default_variant, take 32^3 to 6.1 / 6.4 and
+// 250 x 203 x 187 to 143 / 172.)
 //
 // Node flags: the fused kernels read one byte per node, the node type in bits
 // 0-1 and the BC kinds (BC_FREE) of velocity and T in bits 2 and 3 (0 for

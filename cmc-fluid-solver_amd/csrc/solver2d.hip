@@ -18,16 +18,17 @@
 // Layers other than the state start at zero; their last row and column are
 // never written (the reference reads them from freshly allocated memory).
 //
-// Kernels: one thread per (line, field) runs the Thomas recurrence of
-// Algorithms.h:21-38 in the reference's operation order.  The rows of a
-// work-group's lines are built by all its threads at once into LDS, and each
-// line's recurrence and back substitution then run from there (k2_sweep_lds;
-// lines too long for the LDS keep c', d' in a global scratch, k2_sweep), so a
-// sweep costs about one division chain per row of its longest line.  With one
-// inner iteration a direction is a copy and the sweep, which writes the
-// direction's layers itself.  Copies, merges and the divergence sum are
-// elementwise; the first G Picard iterations of a step, which run whatever
-// their error, are queued back to back and their errors read once.
+// Kernels: the Thomas recurrence of Algorithms.h:21-38 of a (line, field) in the
+// reference's operation order.  The rows of a work-group's lines are built by all
+// its threads at once into LDS; a line's recurrence and back substitution then
+// run in chunks on the lanes of a wavefront, which start early and check one
+// another (k2_sweep_chunks), or, for lines that this does not suit, on one lane
+// (k2_sweep_lds; lines too long for the LDS keep c', d' in a global scratch,
+// k2_sweep).  With one inner iteration a Picard iteration is the two sweeps,
+// which write the directions' layers themselves, and one elementwise kernel for
+// the merge, the next copies and the divergence sums (k2_merge_div).  The first G
+// Picard iterations of a step, which run whatever their error, are queued back
+// to back and their errors read once.
 #pragma clang fp contract(off)
 
 #include "cmcx_internal.h"
