@@ -448,8 +448,8 @@ def stable2d_workload(steps: int = 2):
     viscosity 0.05, density 1000, FP64): the first steps of its driver loop
     (Prepare(t), UpdateBoundaries, TimeStep) on the GPU, grid built on the GPU,
     and the same steps of the oracle on the host; states compared bit for bit.
-    The relaxation is bound by its chain of nx + ny + 1 barrier-separated
-    wavefront steps per sweep, not by HBM or MFMA."""
+    The relaxation is bound by the instructions that one compute unit issues
+    (sweeps in flight on anti-diagonal fronts), not by HBM or MFMA."""
     import oracle_lib
     from cmcx.geometry import Grid2D
     from cmcx.params import FluidParams
@@ -498,7 +498,7 @@ def stable2d_workload(steps: int = 2):
         "cpu_us_per_sweep": cpu_s / sweeps * 1e6,
         "cpu_kind": "port (oracle, 1 thread; the reference's relaxation is serial)",
         "bitwise_equal_to_oracle": same,
-        "bound": "nx + ny + 1 barrier-separated wavefront steps per sweep, sweeps in groups of up to 8 in one work-group",
+        "bound": "instruction issue of one compute unit: sweeps in flight on anti-diagonal fronts, one barrier per step",
     }
 
 
