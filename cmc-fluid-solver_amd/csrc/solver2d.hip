@@ -240,8 +240,8 @@ __global__ void k2_sweep(int nsys, const Sys2* __restrict__ sys, int nx, int ny,
 // is eliminated (a thread's global loads would instead queue behind its own
 // scratch stores: one counter covers both on this architecture).
 // mode 0: the solution on every row into `out` (the local result layer);
-// mode 1 (a direction with one inner iteration): the solution into `lt`, `out`
-// and, where given, `t2` on NODE_IN rows off the grid's last row and column, which is what the
+// mode 1 (a direction with one inner iteration): the solution into `lt` and
+// `out` on NODE_IN rows off the grid's last row and column, which is what the
 // direction's copies leave there (SolveDirection, AdiSolver2D.cpp:203-226:
 // the local layer takes the first solve on NODE_IN, the layer and the result
 // are copied out on NODE_IN, both copies skipping the last row and column);
@@ -259,7 +259,7 @@ template <class T, bool DIRX>
 __global__ void __launch_bounds__(kSweepLdsThreads) k2_sweep_lds(
     int nsys, int spw, int nmax, const Sys2* __restrict__ sys, int nx, int ny,
     const uint8_t* __restrict__ type, const uint8_t* __restrict__ bc, L3<T> g, L3<T> lc,
-    L3<T> tl, L3<T> out, L3<T> lt, L3<T> t2, L3<T> dm, int mode, P2 prm) {
+    L3<T> tl, L3<T> out, L3<T> lt, L3<T> dm, int mode, P2 prm) {
     extern __shared__ char smem2[];
     constexpr int R = kSweepBatch;
     const int rs = spw * nmax;  // rows in LDS
@@ -340,14 +340,12 @@ __global__ void __launch_bounds__(kSweepLdsThreads) k2_sweep_lds(
     // (the flag bytes are read in mode 0 too, unused: no load under a branch)
     T* const o1 = out.f[var];
     T* const o2 = mode == 1 ? lt.f[var] : out.f[var];
-    T* const o3 = mode == 1 && t2.f[var] ? t2.f[var] : o2;
     T* const od = dm.f[var];
     auto put = [&](int t, T v, uint8_t f) {
         const int64_t ct = cell(q, t);
         const bool w = mode == 0 || f != 0;
         (w ? o1 : od)[ct] = v;
         (w ? o2 : od)[ct] = v;
-        (w ? o3 : od)[ct] = v;
     };
     T x = dp;
     put(n - 1, x, mf[(n - 1) * spw]);
@@ -1790,8 +1788,11 @@ class Solver2D final : public ISolver2 {
         return (int)std::min<double>(rows, nmax);
     }
 
-    // mode 1: k2_sweep_lds writes lt and out on the NODE_IN rows (a direction
-    // with one inner iteration), else the solution into out
+    // mode 1: the solve writes lt, out and, where given, t2 (a copy of lt that is
+    // kept up to date) on the NODE_IN rows (a direction with one inner iteration),
+    // else the solution into out.  k2_sweep_lds leaves t2 to a copy: a third
+    // store per row lengthens its serial back substitution (FP64 rows of 700: X 389
+    // -> 413 us; of 2000: 4508 -> 4824, where the copy takes 36).
     void sweep_lds(bool dirx, int spw, int mode, L3<T> lc, L3<T> tlc, L3<T> out, L3<T> lt, L3<T> t2 = {}) {
         const int n = dirx ? nrows : ncols, nmax = dirx ? rows_nmax : cols_nmax;
         if (const int early = early_rows(dirx)) {
@@ -1813,13 +1814,14 @@ class Solver2D final : public ISolver2 {
         const dim3 grid((unsigned)((n + spw - 1) / spw), 3);
         if (dirx)
             hipLaunchKernelGGL((k2_sweep_lds<T, true>), grid, dim3(kSweepLdsThreads), lds, st, n,
-                               spw, nmax, d_rows, nx, ny, d_type, d_bc, g, lc, tlc, out, lt, t2, nl,
+                               spw, nmax, d_rows, nx, ny, d_type, d_bc, g, lc, tlc, out, lt, nl,
                                mode, prm);
         else
             hipLaunchKernelGGL((k2_sweep_lds<T, false>), grid, dim3(kSweepLdsThreads), lds, st, n,
-                               spw, nmax, d_cols, nx, ny, d_type, d_bc, g, lc, tlc, out, lt, t2, nl,
+                               spw, nmax, d_cols, nx, ny, d_type, d_bc, g, lc, tlc, out, lt, nl,
                                mode, prm);
         CMCX_LAUNCH_CHECK();
+        if (t2.f[0]) copy(lt, t2, kAll, 0);
     }
 
     void sweep(bool dirx, L3<T> lc, L3<T> lt, L3<T> out) {
