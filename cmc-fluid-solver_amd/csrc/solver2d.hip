@@ -73,7 +73,7 @@ __global__ void k2_copy(int nx, int ny, const uint8_t* __restrict__ type, int ma
 }
 
 // The step's copies of the state on nodes (i < nx-1, j < ny-1) as k2_copy, with
-// both directions' first copies of the Picard layer: d0..d4 <- src.
+// both directions' first copies of the Picard layer: d0..d4 <- src (d4 unless null).
 template <class T>
 __global__ void k2_fan(int nx, int ny, L3<T> src, L3<T> d0, L3<T> d1, L3<T> d2, L3<T> d3, L3<T> d4) {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -87,7 +87,7 @@ __global__ void k2_fan(int nx, int ny, L3<T> src, L3<T> d0, L3<T> d1, L3<T> d2, 
         d1.f[f][q] = v;
         d2.f[f][q] = v;
         d3.f[f][q] = v;
-        d4.f[f][q] = v;
+        if (d4.f[f]) d4.f[f][q] = v;
     }
 }
 
@@ -619,7 +619,8 @@ __global__ void __launch_bounds__(kSweepLdsThreads) k2_sweep_chunks(
 }
 
 // TimeLayer2D::EvalDivError: per-block partial sums of |tx + ty| in the field
-// type and counts; the finish kernel adds them in block order.
+// type and counts; the finish kernel adds them in block order.  The first
+// kDiv2Blocks blocks of a launch take part, whatever its size.
 constexpr int kDiv2Blocks = 256;
 
 template <class T>
@@ -629,7 +630,7 @@ __device__ __forceinline__ void div_part(int nx, int ny, const uint8_t* __restri
     double sum = 0, cnt = 0;
     const int64_t n = (int64_t)(nx - 1) * (ny - 1);
     for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n;
-         q += (int64_t)gridDim.x * blockDim.x) {
+         q += (int64_t)kDiv2Blocks * blockDim.x) {
         const int i = (int)(q / (ny - 1)), j = (int)(q % (ny - 1));
         const int64_t c = (int64_t)i * ny + j;
         if (type[c] == NODE_IN && type[c + ny] == NODE_IN && type[c + 1] == NODE_IN &&
@@ -669,16 +670,17 @@ __global__ void k2_div(int nx, int ny, const uint8_t* __restrict__ type, L3<T> L
 // (merge: (temp + next) / 2), tl and tl2 <- temp everywhere (both directions'
 // next copies of the Picard layer), on nodes (i < nx-1, j < ny-1) as k2_copy, and
 // the partial sums of next's divergence error.  Apart, with the copy before the Y
-// direction, these were four launches of about 4.5 us each.
+// direction, these were four launches of about 4.5 us each.  A cell per thread, in
+// as many blocks as that takes: in the sums' 256 blocks alone the merge of
+// a 2000 x 2000 FP64 grid took 273 us (too few loads in flight), and takes 119 so, a
+// 700 x 700 one 29 and 18.  Without tl2 (null) its cells are not written.
 template <class T>
 __global__ void __launch_bounds__(kBS2) k2_merge_div(int nx, int ny, const uint8_t* __restrict__ type,
                                                      int merge, L3<T> next, L3<T> temp, L3<T> tl, L3<T> tl2,
                                                      T dx, T dy, double* __restrict__ part) {
-    const int64_t n = (int64_t)nx * ny;
-    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n;
-         q += (int64_t)gridDim.x * blockDim.x) {
-        const int i = (int)(q / ny), j = (int)(q % ny);
-        if (i >= nx - 1 || j >= ny - 1) continue;
+    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    // (the cells of a grid that fits the memory fit 32 bits)
+    if (q < (int64_t)(nx - 1) * ny && (int)((uint32_t)q % (uint32_t)ny) < ny - 1) {
         const bool in = type[q] == NODE_IN;
 #pragma unroll
         for (int f = 0; f < 3; f++) {
@@ -688,10 +690,10 @@ __global__ void __launch_bounds__(kBS2) k2_merge_div(int nx, int ny, const uint8
                 temp.f[f][q] = v;
             }
             tl.f[f][q] = v;
-            tl2.f[f][q] = v;
+            if (tl2.f[f]) tl2.f[f][q] = v;
         }
     }
-    div_part<T>(nx, ny, type, next, dx, dy, part);
+    if (blockIdx.x < kDiv2Blocks) div_part<T>(nx, ny, type, next, dx, dy, part);
 }
 
 // One work-group of kDiv2Blocks threads per slot: its partials come into LDS in
@@ -2008,9 +2010,11 @@ class Solver2D final : public ISolver2 {
         if (G < 0 || L < 1) return CMCX_ERR_ARG;
         prm.dt = dt;
         const bool fused = one_pass(L);
+        // the Picard layer's second copy, unless a copy makes it (sweep_lds)
+        const L3<T> second = fused && early_rows(true) ? tl2 : L3<T>{};
         if (fused) {
             hipLaunchKernelGGL((k2_fan<T>), dim3(blocks2(N)), dim3(kBS2), 0, st, nx, ny, cur, next,
-                               half, temp, tl, tl2);
+                               half, temp, tl, second);
             CMCX_LAUNCH_CHECK();
         } else {
             copy(cur, next, kAll, 0);
@@ -2029,11 +2033,11 @@ class Solver2D final : public ISolver2 {
         for (int k = 0; k < batch; k++) {
             if (fused) {
                 // tl and tl2 hold the Picard layer (k2_fan, k2_merge_div); the X
-                // sweep keeps tl2 up to date for the Y sweep
+                // sweep brings tl2 up to date for the Y sweep
                 sweep_lds(true, lds_spw(true), 1, cur, tl, half, temp, tl2);
                 sweep_lds(false, lds_spw(false), 1, half, tl2, next, temp);
-                hipLaunchKernelGGL((k2_merge_div<T>), dim3(kDiv2Blocks), dim3(kBS2), 0, st, nx, ny, d_type,
-                                   k == 0 ? 0 : 1, next, temp, tl, tl2, (T)prm.dx, (T)prm.dy,
+                hipLaunchKernelGGL((k2_merge_div<T>), dim3(std::max<unsigned>(kDiv2Blocks, blocks2(N))), dim3(kBS2), 0,
+                                   st, nx, ny, d_type, k == 0 ? 0 : 1, next, temp, tl, second, (T)prm.dx, (T)prm.dy,
                                    d_part + (int64_t)k * 2 * kDiv2Blocks);
                 CMCX_LAUNCH_CHECK();
             } else {
