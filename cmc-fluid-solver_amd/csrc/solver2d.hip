@@ -1443,8 +1443,8 @@ class Solver2D final : public ISolver2 {
     double* h_err = nullptr;  // their pinned host copy
     static constexpr int kErrSlots = 64;
     int method = CMCX2D_ADI;
-    // Stable solver: next_w, div, q (whole grid and per-row spans), spans and
-    // cell flags of the relaxation, its status words
+    // Stable solver: next_w, q over the whole grid, the relaxation's status words;
+    // of k2s_poisson div, q per row's span, the spans and their cells' flags
     L3<T> nw{};
     T *d_nw = nullptr, *d_dv = nullptr, *d_qf = nullptr, *d_qspan = nullptr;
     T* d_save = nullptr;  // q at the start of a relaxation group
@@ -1457,6 +1457,8 @@ class Solver2D final : public ISolver2 {
     // length, members, boundary wavefronts, boundary list pitch
     int rl_P = 0, rl_rp = 0, rl_D = 0, rl_mw = 1, rl_bw = 0, rl_cpad = 0;
     uint2* d_blist = nullptr;
+    size_t blist_cap = 0;         // its entries
+    std::vector<uint2> h_blist;   // its host copy, read until the stream has passed its upload
     double* d_dvs = nullptr;
     T *d_qpad = nullptr, *d_qsave = nullptr;
     double ptol = 1e-2;            // POISSON_ERR_THRESHOLD (StableSolver2D.h:23)
@@ -1506,8 +1508,9 @@ class Solver2D final : public ISolver2 {
         CMCX_HIP(hipStreamSynchronize(st));
     }
 
-    // PrepareIndices (StableSolver2D.cpp:167-188) for the fixed mask: per row
-    // the span of non-outside cells and the cells' relaxation flags.
+    // PrepareIndices (StableSolver2D.cpp:167-188) for the fixed mask: the lists of
+    // the relaxation that runs on grids of this size (the stream is waited for
+    // before the host's copies are used again, see h_blist).
     void build_relaxation(const uint8_t* t) {
         auto T_ = [&](int i, int j) -> int {
             return (i < 0 || j < 0 || i >= nx || j >= ny) ? (int)NODE_OUT : t[(int64_t)i * ny + j];
@@ -1518,6 +1521,30 @@ class Solver2D final : public ISolver2 {
                     throw std::string("2D Stable: a NODE_IN cell on the grid's edge (" + std::to_string(i) +
                                       ", " + std::to_string(j) + ")");
         if (nx > 512) throw std::string("2D Stable: grids of more than 512 rows (dimx) are not supported");
+        if (!d_pstat) {
+            CMCX_HIP(hipMalloc((void**)&d_nw, sizeof(T) * N * 2));
+            CMCX_HIP(hipMalloc((void**)&d_qf, sizeof(T) * N));
+            CMCX_HIP(hipMemsetAsync(d_nw, 0, sizeof(T) * N * 2, st));
+            nw.f[0] = d_nw;
+            nw.f[1] = d_nw + N;
+            nw.f[2] = temp.f[2];  // never read or written (the step solves u and v only)
+            CMCX_HIP(hipMalloc((void**)&d_pstat, sizeof(int32_t) * 4));
+        }
+        // q in LDS by anti-diagonals where it fits there and a cell's place in
+        // sweep order 16 bits
+        const int rp = (nx + 63) / 64 * 64, smax = std::max(1, std::min(15, (1024 - 64) / rp));
+        int P = std::max(ny + 1, kPoisLag * smax);
+        if (nx > P) P = std::min(nx, (P + 63) / 64 * 64);
+        const int64_t cells = (int64_t)(nx + 2) * P;
+        if (cells * (int64_t)sizeof(T) + 3072 > 160 * 1024 || cells > 0xffff) build_spans(t);
+        else build_fronts(t, P, rp, smax);
+    }
+
+    // k2s_poisson: per row the span of non-outside cells and the cells' flags.
+    void build_spans(const uint8_t* t) {
+        auto T_ = [&](int i, int j) -> int {
+            return (i < 0 || j < 0 || i >= nx || j >= ny) ? (int)NODE_OUT : t[(int64_t)i * ny + j];
+        };
         std::vector<int32_t> sp(3 * (size_t)nx);
         std::vector<uint8_t> fl;
         for (int i = 0; i < nx; i++) {
@@ -1561,15 +1588,8 @@ class Solver2D final : public ISolver2 {
             }
             CMCX_HIP(hipMalloc((void**)&d_doff, sizeof(int32_t) * doff.size()));
             CMCX_HIP(hipMemcpy(d_doff, doff.data(), sizeof(int32_t) * doff.size(), hipMemcpyHostToDevice));
-            CMCX_HIP(hipMalloc((void**)&d_spans, sizeof(int32_t) * sp.size()));
-            CMCX_HIP(hipMalloc((void**)&d_nw, sizeof(T) * N * 2));
             CMCX_HIP(hipMalloc((void**)&d_dv, sizeof(T) * N));
-            CMCX_HIP(hipMalloc((void**)&d_qf, sizeof(T) * N));
-            CMCX_HIP(hipMalloc((void**)&d_pstat, sizeof(int32_t) * 4));
-            CMCX_HIP(hipMemsetAsync(d_nw, 0, sizeof(T) * N * 2, st));
-            nw.f[0] = d_nw;
-            nw.f[1] = d_nw + N;
-            nw.f[2] = temp.f[2];  // never read or written (the step solves u and v only)
+            CMCX_HIP(hipMalloc((void**)&d_spans, sizeof(int32_t) * sp.size()));
         }
         CMCX_HIP(hipMalloc((void**)&d_fspan, std::max(S, 1)));
         CMCX_HIP(hipMalloc((void**)&d_qspan, sizeof(T) * std::max(S, 1)));
@@ -1577,35 +1597,25 @@ class Solver2D final : public ISolver2 {
         CMCX_HIP(hipMemcpyAsync(d_spans, sp.data(), sizeof(int32_t) * sp.size(), hipMemcpyHostToDevice, st));
         if (S) CMCX_HIP(hipMemcpyAsync(d_fspan, fl.data(), S, hipMemcpyHostToDevice, st));
         CMCX_HIP(hipStreamSynchronize(st));
-        build_fronts(t);
     }
 
-    // Layout and boundary lists of k2s_poisson_lds, when its q fits the LDS and a
-    // cell's place in sweep order 16 bits.
-    void build_fronts(const uint8_t* t) {
-        const int rp = (nx + 63) / 64 * 64, smax = std::max(1, std::min(15, (1024 - 64) / rp));
-        int P = std::max(ny + 1, kPoisLag * smax);
-        if (nx > P) P = std::min(nx, (P + 63) / 64 * 64);
-        const int64_t cells = (int64_t)(nx + 2) * P;
-        if (cells * (int64_t)sizeof(T) + 3072 > 160 * 1024 || cells > 0xffff) return;
+    // k2s_poisson_lds: its layout and boundary lists.  The arrays are kept from
+    // grid to grid: allocated anew for each, beside the spans that this relaxation
+    // does not read, they took SetGrid on a 120 x 135 grid to 197 us; kept, it takes 92.
+    void build_fronts(const uint8_t* t, int P, int rp, int smax) {
         auto T_ = [&](int i, int j) -> int {
             return (i < 0 || j < 0 || i >= nx || j >= ny) ? (int)NODE_OUT : t[(int64_t)i * ny + j];
         };
-        std::vector<std::vector<uint2>> lists(P);
-        int cmax = 1;
-        for (int i = 0; i < nx; i++)
-            for (int j = 0; j < ny; j++) {
-                const int ty = T_(i, j), x = j + 1;
-                if (ty != NODE_BOUND && ty != NODE_VALVE) continue;
-                uint32_t w = kBValid | (uint32_t)(i * P + x);
-                if (T_(i - 1, j) == NODE_IN) w |= 1u << 16;
-                if (T_(i + 1, j) == NODE_IN) w |= 1u << 17;
-                if (T_(i, j - 1) == NODE_IN) w |= 1u << 18;
-                if (T_(i, j + 1) == NODE_IN) w |= 1u << 19;
-                auto& l = lists[(i + x) % P];
-                l.push_back(uint2{w, (uint32_t)i | (uint32_t)((i + x) / P) << 16});
-                cmax = std::max(cmax, (int)l.size());
-            }
+        std::vector<int> len(P, 0);
+        auto each = [&](auto&& cell) {
+            for (int i = 0; i < nx; i++)
+                for (int j = 0; j < ny; j++) {
+                    const int ty = t[(int64_t)i * ny + j];
+                    if (ty == NODE_BOUND || ty == NODE_VALVE) cell(i, j);
+                }
+        };
+        each([&](int i, int j) { len[(i + j + 1) % P]++; });
+        const int cmax = std::max(1, *std::max_element(len.begin(), len.end()));
         // sweeps per slice as the row length allows; as many slices as leave the
         // boundary wavefronts a lane for every boundary cell of a front (at
         // least half of them otherwise)
@@ -1618,17 +1628,32 @@ class Solver2D final : public ISolver2 {
             if (64 * bw / D >= cmax) break;
         }
         const int epm = 64 * bw / D, cpad = (cmax + epm - 1) / epm * epm;
-        std::vector<uint2> bl((size_t)P * cpad, uint2{0, 0});
-        for (int q = 0; q < P; q++) std::copy(lists[q].begin(), lists[q].end(), bl.begin() + (size_t)q * cpad);
-        hipFree(d_blist);
-        d_blist = nullptr;
-        CMCX_HIP(hipMalloc((void**)&d_blist, sizeof(uint2) * bl.size()));
-        CMCX_HIP(hipMemcpy(d_blist, bl.data(), sizeof(uint2) * bl.size(), hipMemcpyHostToDevice));
-        if (!d_dvs) {
+        CMCX_HIP(hipStreamSynchronize(st));  // h_blist on its way, d_blist in use
+        h_blist.assign((size_t)P * cpad, uint2{0, 0});
+        std::fill(len.begin(), len.end(), 0);
+        each([&](int i, int j) {
+            const int x = j + 1, q = (i + x) % P;
+            uint32_t w = kBValid | (uint32_t)(i * P + x);
+            if (T_(i - 1, j) == NODE_IN) w |= 1u << 16;
+            if (T_(i + 1, j) == NODE_IN) w |= 1u << 17;
+            if (T_(i, j - 1) == NODE_IN) w |= 1u << 18;
+            if (T_(i, j + 1) == NODE_IN) w |= 1u << 19;
+            h_blist[(size_t)q * cpad + len[q]++] = uint2{w, (uint32_t)i | (uint32_t)((i + x) / P) << 16};
+        });
+        if (!d_qsave) {
+            const int64_t cells = (int64_t)(nx + 2) * P;
             CMCX_HIP(hipMalloc((void**)&d_dvs, sizeof(double) * (P + kDvRows) * rp));
             CMCX_HIP(hipMalloc((void**)&d_qpad, sizeof(T) * cells));
             CMCX_HIP(hipMalloc((void**)&d_qsave, sizeof(T) * cells));
         }
+        if (h_blist.size() > blist_cap) {
+            uint2* p = nullptr;
+            CMCX_HIP(hipMalloc((void**)&p, sizeof(uint2) * h_blist.size()));
+            hipFree(d_blist);
+            d_blist = p;
+            blist_cap = h_blist.size();
+        }
+        CMCX_HIP(hipMemcpyAsync(d_blist, h_blist.data(), sizeof(uint2) * h_blist.size(), hipMemcpyHostToDevice, st));
         rl_P = P;
         rl_rp = rp;
         rl_D = D;
