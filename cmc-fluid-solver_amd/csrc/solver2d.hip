@@ -1571,16 +1571,9 @@ class Solver2D final : public ISolver2 {
             fl.push_back(0);
         }
         fl.push_back(0);  // one more guard: the last row's reads stay inside
-        // spans, flags and q per span (sized by the mask); the rest once
-        CMCX_HIP(hipStreamSynchronize(st));
-        hipFree(d_fspan);
-        hipFree(d_qspan);
-        hipFree(d_save);
-        d_fspan = nullptr;
-        d_qspan = nullptr;
-        d_save = nullptr;
-        S = (int)fl.size();
-        if (!d_spans) {
+        // the arrays once, for spans as long as they can be
+        if (!d_save) {
+            const size_t most = (size_t)nx * (ny + 2) + 1;
             std::vector<int32_t> doff(nx + ny);
             for (int d = 0, o = 0; d < nx + ny; d++) {
                 doff[d] = o;
@@ -1590,12 +1583,13 @@ class Solver2D final : public ISolver2 {
             CMCX_HIP(hipMemcpy(d_doff, doff.data(), sizeof(int32_t) * doff.size(), hipMemcpyHostToDevice));
             CMCX_HIP(hipMalloc((void**)&d_dv, sizeof(T) * N));
             CMCX_HIP(hipMalloc((void**)&d_spans, sizeof(int32_t) * sp.size()));
+            CMCX_HIP(hipMalloc((void**)&d_fspan, most));
+            CMCX_HIP(hipMalloc((void**)&d_qspan, sizeof(T) * most));
+            CMCX_HIP(hipMalloc((void**)&d_save, sizeof(T) * most));
         }
-        CMCX_HIP(hipMalloc((void**)&d_fspan, std::max(S, 1)));
-        CMCX_HIP(hipMalloc((void**)&d_qspan, sizeof(T) * std::max(S, 1)));
-        CMCX_HIP(hipMalloc((void**)&d_save, sizeof(T) * std::max(S, 1)));
+        S = (int)fl.size();
         CMCX_HIP(hipMemcpyAsync(d_spans, sp.data(), sizeof(int32_t) * sp.size(), hipMemcpyHostToDevice, st));
-        if (S) CMCX_HIP(hipMemcpyAsync(d_fspan, fl.data(), S, hipMemcpyHostToDevice, st));
+        CMCX_HIP(hipMemcpyAsync(d_fspan, fl.data(), S, hipMemcpyHostToDevice, st));
         CMCX_HIP(hipStreamSynchronize(st));
     }
 
@@ -1675,15 +1669,7 @@ class Solver2D final : public ISolver2 {
                 return CMCX_ERR_ARG;
             }
         if (method == CMCX2D_STABLE) build_relaxation(t);
-        else {
-            CMCX_HIP(hipStreamSynchronize(st));
-            hipFree(d_rows);
-            hipFree(d_cols);
-            hipFree(scratch);
-            d_rows = d_cols = nullptr;
-            scratch = nullptr;
-            build_systems(t);
-        }
+        else build_systems(t);
         CMCX_HIP(hipMemcpyAsync(d_type, t, N, hipMemcpyHostToDevice, st));
         CMCX_HIP(hipMemcpyAsync(d_bc, bc, N, hipMemcpyHostToDevice, st));
         std::vector<T> h(N);
@@ -1722,7 +1708,8 @@ class Solver2D final : public ISolver2 {
         hipFree(d_pstat);
     }
 
-    // AdiSolver2D::CreateSegments (the mask is fixed, so once).
+    // AdiSolver2D::CreateSegments, for each new mask.  Types that are refused, or a
+    // failed allocation, leave the lists there were.
     void build_systems(const uint8_t* t) {
         auto T_ = [&](int i, int j) { return t[(int64_t)i * ny + j]; };
         std::vector<Sys2> rows, cols;
@@ -1752,22 +1739,41 @@ class Solver2D final : public ISolver2 {
             if (s.b - s.a0 + 1 < 2) throw std::string("2D: a line system shorter than 2 nodes");
         for (const Sys2& s : cols)
             if (s.b - s.a1 + 1 < 2) throw std::string("2D: a line system shorter than 2 nodes");
+        const int64_t nsys = std::max<int64_t>(std::max(rows.size(), cols.size()), 1);
+        const int64_t half = (int64_t)std::max(nx, ny) * 3 * nsys;
+        Sys2 *nr = nullptr, *nc = nullptr;
+        T* ns = nullptr;
+        try {
+            if (!rows.empty()) {
+                CMCX_HIP(hipMalloc((void**)&nr, sizeof(Sys2) * rows.size()));
+                CMCX_HIP(hipMemcpy(nr, rows.data(), sizeof(Sys2) * rows.size(), hipMemcpyHostToDevice));
+            }
+            if (!cols.empty()) {
+                CMCX_HIP(hipMalloc((void**)&nc, sizeof(Sys2) * cols.size()));
+                CMCX_HIP(hipMemcpy(nc, cols.data(), sizeof(Sys2) * cols.size(), hipMemcpyHostToDevice));
+            }
+            if (half > sc_half) CMCX_HIP(hipMalloc((void**)&ns, sizeof(T) * 2 * half));
+            CMCX_HIP(hipStreamSynchronize(st));  // the old lists' last reader
+        } catch (...) {
+            hipFree(nr);
+            hipFree(nc);
+            hipFree(ns);
+            throw;
+        }
+        hipFree(d_rows);
+        hipFree(d_cols);
+        d_rows = nr;
+        d_cols = nc;
+        if (ns) {
+            hipFree(scratch);
+            scratch = ns;
+            sc_half = half;
+        }
         nrows = (int)rows.size();
         ncols = (int)cols.size();
         rows_nmax = cols_nmax = 0;
         for (const Sys2& s : rows) rows_nmax = std::max(rows_nmax, s.b - s.a0 + 1);
         for (const Sys2& s : cols) cols_nmax = std::max(cols_nmax, s.b - s.a1 + 1);
-        if (nrows) {
-            CMCX_HIP(hipMalloc((void**)&d_rows, sizeof(Sys2) * nrows));
-            CMCX_HIP(hipMemcpy(d_rows, rows.data(), sizeof(Sys2) * nrows, hipMemcpyHostToDevice));
-        }
-        if (ncols) {
-            CMCX_HIP(hipMalloc((void**)&d_cols, sizeof(Sys2) * ncols));
-            CMCX_HIP(hipMemcpy(d_cols, cols.data(), sizeof(Sys2) * ncols, hipMemcpyHostToDevice));
-        }
-        const int64_t nsys = std::max(nrows, ncols);
-        sc_half = (int64_t)std::max(nx, ny) * 3 * std::max<int64_t>(nsys, 1);
-        CMCX_HIP(hipMalloc((void**)&scratch, sizeof(T) * 2 * sc_half));
     }
 
     void copy(L3<T> src, L3<T> dst, int mask, int merge) {
