@@ -27,10 +27,15 @@ struct HipError {
     std::string where;
 };
 
+// A failed call's error is taken from the runtime, which would give it to the next
+// launch check of the thread, another solver's too.
 #define CMCX_HIP(expr)                                                            \
     do {                                                                          \
         hipError_t _e = (expr);                                                   \
-        if (_e != hipSuccess) throw ::cmcx::HipError{_e, std::string(#expr)};     \
+        if (_e != hipSuccess) {                                                   \
+            (void)hipGetLastError();                                              \
+            throw ::cmcx::HipError{_e, std::string(#expr)};                       \
+        }                                                                         \
     } while (0)
 
 #define CMCX_LAUNCH_CHECK()                                                       \
