@@ -183,6 +183,7 @@ class Solver final : public ISolver {
         T* work = nullptr;     // xbar, tbar, state-adjoint sum, lam, node-value gradient, final state
         double* pp = nullptr;  // per-block parameter partials
         uint16_t* nmask = nullptr;  // node words of the pointwise kernel
+        bool ready = false;         // work, pp, nmask and the tiles are there
         int32_t* tiles[3] = {nullptr, nullptr, nullptr};
         int64_t ntiles[3] = {0, 0, 0};
         int ltiles[3] = {0, 0, 0};
@@ -1170,10 +1171,14 @@ class Solver final : public ISolver {
             set_error("adjoint: axes of at most 256 nodes and no BC_FREE node shared by two segments");
             return CMCX_ERR_UNSUPPORTED;
         }
-        const int nck = (steps + every - 1) / every;
+        // (from here on the last recording is gone, also if an allocation fails)
+        adj.recorded = false;
+        adj.invalid_why = "an adjoint_forward that failed";
+        const int nck = (steps - 1) / every + 1;
         if (nck > adj.nck) {
             hipFree(adj.ck);
             adj.ck = nullptr;
+            adj.nck = 0;
             CMCX_HIP(hipMalloc((void**)&adj.ck, sizeof(T) * 4 * NT * nck));
             adj.nck = nck;
         }
@@ -1229,11 +1234,12 @@ class Solver final : public ISolver {
         if (need > adj.tape_layers || adj.tape_G != adj.G) {
             hipFree(adj.tape);
             adj.tape = nullptr;
+            adj.tape_layers = 0;
+            adj.tape_values = false;
+            adj.holds[0] = adj.holds[1] = -1;
             CMCX_HIP(hipMalloc((void**)&adj.tape, sizeof(T) * (4 * NT * need + kSlack)));
             adj.tape_layers = need;
             adj.tape_G = adj.G;
-            adj.tape_values = false;
-            adj.holds[0] = adj.holds[1] = -1;
         }
         adj.nbuf = nbuf;
         if (!adj.tape_values) {
@@ -1309,13 +1315,15 @@ class Solver final : public ISolver {
         const Geom& g = grids[0].g;
         const int64_t per = 1 + 6 * (int64_t)adj.G;
         ensure_tape();
-        if (!adj.work) {
-            CMCX_HIP(hipMalloc((void**)&adj.work, sizeof(T) * (4 * NT * 6 + kSlack)));
-            CMCX_HIP(hipMalloc((void**)&adj.pp, sizeof(double) * 4 * adj_point_blocks()));
-            CMCX_HIP(hipMalloc((void**)&adj.nmask, sizeof(uint16_t) * g.N));
+        if (!adj.ready) {  // (what an earlier, failed call allocated is kept)
+            if (!adj.work) CMCX_HIP(hipMalloc((void**)&adj.work, sizeof(T) * (4 * NT * 6 + kSlack)));
+            if (!adj.pp) CMCX_HIP(hipMalloc((void**)&adj.pp, sizeof(double) * 4 * adj_point_blocks()));
+            if (!adj.nmask) CMCX_HIP(hipMalloc((void**)&adj.nmask, sizeof(uint16_t) * g.N));
             for (int a = 0; a < 3; a++)
-                build_adj_tiles(h_type.data(), g, a, adj_lpg<T>(g), &adj.tiles[a], &adj.ntiles[a],
-                                &adj.ltiles[a]);
+                if (!adj.tiles[a])
+                    build_adj_tiles(h_type.data(), g, a, adj_lpg<T>(g), &adj.tiles[a], &adj.ntiles[a],
+                                    &adj.ltiles[a]);
+            adj.ready = true;
         }
         Layer4<T> XB = lay(adj.work, 0), GB = lay(adj.work, 4), FIN = lay(adj.work, 5);
         copy_layer(FIN, cur);
@@ -1336,7 +1344,7 @@ class Solver final : public ISolver {
         // own) while interval i is reversed on the solver's stream; events
         // order a reverse after its interval's recompute, and a recompute
         // after the reverse that last used its buffer.
-        const int nseg = (adj.steps + adj.every - 1) / adj.every;
+        const int nseg = (adj.steps - 1) / adj.every + 1;
         const int nb = adj.nbuf;
         if (!adj.fs) CMCX_HIP(hipStreamCreateWithFlags(&adj.fs, hipStreamNonBlocking));
         std::vector<hipEvent_t> recd(nseg, nullptr), revd(nseg, nullptr);
