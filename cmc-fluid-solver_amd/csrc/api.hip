@@ -840,19 +840,31 @@ class Solver final : public ISolver {
         return CMCX_OK;
     }
 
-    // Whether a kernel of this device may write every (non-null) address as
-    // elements of the field type; other memory is left to the runtime's copies.
-    static bool on_this_device(std::initializer_list<const void*> ptrs) {
+    // Whether a kernel of this device may write `bytes` at every (non-null) address
+    // as elements of the field type.  Other memory, and arrays that end before, are
+    // left to the runtime's copies, which know the one and refuse the other.
+    static bool on_this_device(std::initializer_list<const void*> ptrs, size_t bytes) {
         int dev = -1;
         if (hipGetDevice(&dev) != hipSuccess) return false;
+        uintptr_t lo = 0, hi = 0;  // the allocation of the address before
         for (const void* q : ptrs) {
             if (!q) continue;
-            hipPointerAttribute_t a;
-            if (hipPointerGetAttributes(&a, q) != hipSuccess) {
-                (void)hipGetLastError();  // not an address the runtime knows
-                return false;
+            const uintptr_t at = (uintptr_t)q;
+            if (at < lo || at >= hi) {
+                hipPointerAttribute_t a;
+                hipDeviceptr_t base = nullptr;
+                size_t size = 0;
+                if (hipPointerGetAttributes(&a, q) != hipSuccess ||
+                    hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)q) != hipSuccess) {
+                    (void)hipGetLastError();  // not an address the runtime knows
+                    return false;
+                }
+                if (a.type != hipMemoryTypeDevice || a.device != dev) return false;
+                lo = (uintptr_t)base;
+                hi = lo + size;
+                if (at < lo || at >= hi) return false;
             }
-            if (a.type != hipMemoryTypeDevice || a.device != dev || (uintptr_t)q % sizeof(T)) return false;
+            if (at % sizeof(T) || bytes > hi - at) return false;
         }
         return true;
     }
@@ -862,7 +874,7 @@ class Solver final : public ISolver {
         const int64_t N = Gr.g.N, o = Gr.off;
         hipMemcpyKind k = device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
         void* dst[4] = {u, v, w, Tt};
-        if (device && on_this_device({u, v, w, p, Tt})) {
+        if (device && on_this_device({u, v, w, p, Tt}, sizeof(T) * N)) {
             Layer4<T> to;
             for (int f = 0; f < 4; f++) to.f[f] = (T*)dst[f];
             launch_read_state<T>(shifted(cur, o), to, (T*)p, (T)Gr.prm.v_T, N, st);
