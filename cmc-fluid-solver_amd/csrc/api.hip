@@ -406,7 +406,10 @@ class Solver final : public ISolver {
                     set_error("fused path: grid lines longer than supported");
                     return CMCX_ERR_UNSUPPORTED;
                 }
-        if (p != path || m != merge_order) invalidate_recording("set_options");
+        if (p != path || m != merge_order) {
+            invalidate_recording("set_options");
+            adj.tape_values = false;
+        }
         path = p;
         merge_order = m;
         clear_graphs();
@@ -1235,9 +1238,14 @@ class Solver final : public ISolver {
     // Tape of the checkpoint intervals: two buffers when the rollout has more
     // than one interval (the backward pass recomputes one interval while it
     // reverses the next), else one.  The Picard-layer slots hold the node
-    // values on non-IN nodes (the forward's temp holds the boundary-filled state
-    // there, and the sweeps write NODE_IN nodes only), put there when the tape
-    // is allocated and again after new node values.
+    // values on BOUND and VALVE nodes, as the forward's temp holds the
+    // boundary-filled state there: put there when the tape is allocated, and again
+    // after new node values and other options.  In between they stay: the
+    // strided sweeps and the per-segment ones write NODE_IN nodes only, and the
+    // fused Z sweep, which writes its lines whole, carries over its input's values,
+    // the boundary-filled state's or the slot before's.  On NODE_OUT nodes it leaves
+    // whatever the state holds there, which nothing reads (no NODE_IN node has
+    // such a neighbour).
     void ensure_tape() {
         const int64_t per = 1 + 6 * (int64_t)adj.G;
         const int64_t nsteps_tape = std::min(adj.every, adj.steps);
