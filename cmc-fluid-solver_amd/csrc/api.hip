@@ -155,6 +155,13 @@ class Solver final : public ISolver {
     // resampled output nodes on their way to the host (T, then u, v, w), at most
     // kOutChunk of them
     static constexpr int64_t kOutChunk = 1 << 20;
+    // output nodes per node from which a layer is resampled on the host: more bytes
+    // would then cross as resampled nodes, into the program's pages, than as the
+    // layer.  On the device / on the host, us, into pages in use and into new
+    // ones: FP64 48^3 1 node per node 250 / 381, 836 / 1262; 2 517 / 539, 1109 / 1385; 4
+    // 1065 / 860, 1906 / 1818; 9 2384 / 1734, 3320 / 3142; FP32 32^3 2 96 / 172, 286 / 332;
+    // 4 202 / 260, 645 / 545; 9 441 / 475, 1455 / 1079.
+    static constexpr int64_t kOutFine = 2;
     double* out_buf = nullptr;
     int64_t out_cap = 0;
     // HIP graphs of whole steps, per (boundary fill, dt, G, L, state buffer)
@@ -940,8 +947,27 @@ class Solver final : public ISolver {
             launch_fill_typed<T>(g, d_type + Gr.off, NODE_OUT, shifted(next, Gr.off), miss, miss, miss, miss, st);
             out_fill[sel] |= (uint8_t)(1 << state_buffer(next));
         }
-        // resampled on the device, kOutChunk nodes at a time
-        const int64_t n = (int64_t)ox * oy * oz, cap = std::min(n, kOutChunk);
+        const int64_t n = (int64_t)ox * oy * oz, N = g.N;
+        // resampled on the device, kOutChunk nodes at a time, or, if that gives over
+        // kOutFine nodes for one of the layer, on the host
+        if (n > kOutFine * N) {
+            std::vector<T> h[4];
+            for (int f = 0; f < 4; f++) {
+                h[f].resize(N);
+                CMCX_HIP(hipMemcpyAsync(h[f].data(), next.f[f] + Gr.off, sizeof(T) * N, hipMemcpyDeviceToHost, st));
+            }
+            CMCX_HIP(hipStreamSynchronize(st));
+            int64_t q = 0;
+            for (int64_t i = 0; i < ox; i++)
+                for (int64_t j = 0; j < oy; j++)
+                    for (int64_t k = 0; k < oz; k++, q++) {
+                        const int64_t src = (i * g.nx / ox) * g.sx + (j * g.ny / oy) * g.sy + k * g.nz / oz;
+                        for (int f = 0; f < 3; f++) ((T*)vel)[3 * q + f] = h[f][src];
+                        Tout[q] = (double)h[3][src];
+                    }
+            return CMCX_OK;
+        }
+        const int64_t cap = std::min(n, kOutChunk);
         if (cap > out_cap) {
             hipFree(out_buf);
             out_buf = nullptr;
