@@ -297,11 +297,14 @@ class Solver final : public ISolver {
     void upload_free_list() {
         std::vector<uint32_t> fl;
         for (const Grid& G : grids)
-            for (int64_t k = 0; k < G.g.N; k++) {
-                const int64_t i = G.off + k;
-                const uint8_t t = h_type[i];
-                if ((t == NODE_BOUND || t == NODE_VALVE) && (h_bcv[i] == BC_FREE || h_bct[i] == BC_FREE))
-                    fl.push_back((uint32_t)i);
+            for (int64_t row = G.off; row < G.off + G.g.N; row += G.g.nz) {
+                // (most z lines have none)
+                if (!std::memchr(&h_bcv[row], BC_FREE, G.g.nz) && !std::memchr(&h_bct[row], BC_FREE, G.g.nz)) continue;
+                for (int64_t i = row; i < row + G.g.nz; i++) {
+                    const uint8_t t = h_type[i];
+                    if ((t == NODE_BOUND || t == NODE_VALVE) && (h_bcv[i] == BC_FREE || h_bct[i] == BC_FREE))
+                        fl.push_back((uint32_t)i);
+                }
             }
         n_bvfree = (int64_t)fl.size();
         if (n_bvfree)

@@ -73,6 +73,7 @@
 #include "line_solve.h"
 
 #include <algorithm>
+#include <cstring>
 #include <stdexcept>
 
 namespace cmcx {
@@ -1146,9 +1147,13 @@ int shared_free_axes(const uint8_t* t, const uint8_t* bv, const uint8_t* bt, con
     const int64_t str[3] = {g.sx, g.sy, 1};
     const int dim[3] = {g.nx, g.ny, g.nz};
     for (int x = 0; x < g.nx; x++)
-        for (int y = 0; y < g.ny; y++)
+        for (int y = 0; y < g.ny; y++) {
+            // most z lines have no free node: a search of each line's kinds, where a
+            // look at every node takes a tenth of set_boundary on a 128^3 grid
+            const int64_t row = x * g.sx + y * g.sy;
+            if (!std::memchr(bv + row, BC_FREE, g.nz) && !std::memchr(bt + row, BC_FREE, g.nz)) continue;
             for (int z = 0; z < g.nz; z++) {
-                int64_t c = x * g.sx + y * g.sy + z;
+                const int64_t c = row + z;
                 if (t[c] == NODE_IN || (bv[c] != BC_FREE && bt[c] != BC_FREE)) continue;
                 const int pos[3] = {x, y, z};
                 for (int a = 0; a < 3; a++)
@@ -1156,6 +1161,7 @@ int shared_free_axes(const uint8_t* t, const uint8_t* bv, const uint8_t* bt, con
                         t[c + str[a]] == NODE_IN)
                         mask |= 1 << a;
             }
+        }
     return mask;
 }
 
