@@ -24,9 +24,10 @@
 // the X sweep that follows covers the node it overwrites it, here too.  The
 // strided (X, Y) sweeps store segment rows only, as the reference (storing the
 // other rows as well costs them more in bytes than it gains).  When a launch's
-// 16 fields exceed the memory-side cache, all stores are non-temporal
-// (kStoreStream): written lines would otherwise evict lines that the sweep
-// still reads (the Picard layer for the merge, the cross-line rows).
+// 16 fields exceed the memory-side cache and every z line is whole 128-byte lines,
+// stores are non-temporal (kStoreStream; not in Z sweeps whose lanes hold more
+// than one 16-byte vector): written lines would otherwise evict lines that the
+// sweep still reads (the Picard layer for the merge, the cross-line rows).
 //
 // Each line is solved by the chunked partition method of line_solve.h (chunks
 // of M rows per lane, reduced system of 2 rows per chunk, compacted by one
@@ -45,10 +46,10 @@
 // takes its differences from the advection term.  With the rows handled one by
 // one, selects for every role and a 64-bit address per access (over 300 per
 // row) the sweeps took, on 128-byte tiles, X / Y / Z in us: 32^3 FP32 9.3 / 9.9 /
-// 5.0, so 6.6 / 7.5 / 3.8; 64^3 11.2 / 12.3 / 9.2, so 8.3 / 10.5 / 7.6; 250 x 203
-// x 187 167 / 202 / 142, so 152 / 190 / 142; 256^3 267 / 303 / 187, so 261 / 272
-// / 185.  (Tiles chosen by size, fused_default_variant, take 32^3 to 6.1 / 6.4 and
-// 250 x 203 x 187 to 143 / 172.)
+// 5.0, so 6.8 / 7.4 / 4.5; 64^3 11.2 / 12.3 / 9.2, so 8.0 / 10.5 / 7.8; 250 x 203
+// x 187 167 / 202 / 142, so 152 / 192 / 138; 256^3 267 / 303 / 187, so 261 / 272
+// / 183.  (Tiles chosen by size, fused_default_variant, take 32^3 to 6.2 / 6.4 and
+// 250 x 203 x 187 to 142 / 174.)
 //
 // Node flags: the fused kernels read one byte per node, the node type in bits
 // 0-1 and the BC kinds (BC_FREE) of velocity and T in bits 2 and 3 (0 for
@@ -59,10 +60,11 @@
 //
 // Layouts:
 //   strided lines (X and Y sweeps): a work-group owns LPG consecutive z lines
-//     (LPG * sizeof(T) = 128 bytes: every row access of a lane group is one
-//     cache line) and all rows; lane group g of wave w owns chunk w*(64/LPG)+g.
-//   contiguous lines (Z sweep): 32 lanes per line, two lines per wavefront,
-//     lane l owns rows [l*M, l*M+M) (vector loads).
+//     (LPG * sizeof(T) = 128 bytes, every row access of a lane group one cache
+//     line; 64 or 32 where those are too few work-groups) and all rows; lane group
+//     g of wave w owns chunk w*(64/LPG)+g.
+//   contiguous lines (Z sweep): 32 or 64 lanes per line, two lines or one per
+//     wavefront, lane l owns rows [l*M, l*M+M) (vector loads).
 // A launch covers a batch of independent grids stored back to back in the flat
 // field arrays: each work-group reads its grid's geometry and coefficients from
 // a descriptor table (one grid is a batch of one).
@@ -438,10 +440,7 @@ __host__ __device__ constexpr int keep_row_pitch(int lpg, int m) {
 }
 
 // ---------------------------------------------------------------------------
-// Strided lines (X or Y sweep).  A work-group owns LPG consecutive z lines and
-// every row of them (MAXT = 32 * LPG threads for lines of up to 256 rows in
-// chunks of M = 8); MINW is the occupancy the register allocation must allow
-// (waves per SIMD), so that two half-width work-groups can share a CU.
+// A strided work-group's tile (fused_strided_kernel below).
 template <class T, int AXIS, int M, int LPG, bool KEEP, bool BSYNC>
 __device__ __forceinline__ void strided_tile(const InstDesc<T>* __restrict__ insts, T three_dt,
                                              const uint8_t* __restrict__ type, const T* const* gval,
@@ -468,8 +467,8 @@ __device__ __forceinline__ void strided_tile(const InstDesc<T>* __restrict__ ins
     // reduced solve treats them as one line.  With one grid (`one`) its
     // descriptor is read beside the item, not after it, and with one tile per
     // item no division finds the tile: on small grids the kernel is little more
-    // than this chain of loads and the one that follows (64^3 FP32 X 7.9 -> 7.6,
-    // Y 9.7 -> 9.5 us; the Z sweep gains nothing from it).
+    // than this chain of loads and the one that follows (64^3 FP32 X 7.9 -> 7.7,
+    // Y 9.7 -> 9.6 us; the Z sweep gains nothing from it).
     const int b = (int)xcd_remap(blockIdx.x, gridDim.x);
     const int32_t* item = work + (int64_t)b * (kmax + 1);
     int inst = 0;
@@ -883,7 +882,12 @@ bool fused_variant_ok(int n, int v) {
 // lines of at most 64 nodes take 32-byte tiles of 4-row chunks (24^3 and 32^3:
 // FP32 step 80 / 73 us, FP64 101 / 92), longer ones 32-byte tiles of 8-row chunks
 // up to 80 and 64-byte tiles up to 128 (FP32 189 x 39 x 40, 78 X tiles: 164 / 152
-// us; FP64 35 x 158 x 33, 105 Y tiles: 194 / 177).  Otherwise 128-byte tiles; the Picard
+// us; FP64 35 x 158 x 33, 105 Y tiles: 194 / 177).  Otherwise 128-byte tiles, though
+// not always the best: how evenly they fall on the CUs is not looked at.  Of a few
+// dozen shapes measured in all variants, these lost most, us per step with the
+// default and with the best one: FP64 160 x 40 x 100 (280 X tiles) 322 / 283 with 64-byte
+// parked, 105 x 139 x 158 (1050 Y tiles) 1019 / 969, 223 x 138 x 213 3044 / 2914; FP32
+// 234 x 86 x 119 440 / 416, 96^3 180 / 175.  The autotuner finds them.  The Picard
 // layer is parked in LDS for the merge once its four fields are 8 MiB, a quarter
 // of the chip's L2: the second read of a smaller one hits there (64^3 FP32: 112 us
 // read again, 115 parked), that of a larger one goes further out (FP32 128^3

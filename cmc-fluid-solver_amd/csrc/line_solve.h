@@ -170,6 +170,14 @@ __device__ __forceinline__ double lane_next(double x) {
 // are decoupled after 0 to 2 of the 5 steps that 32 chunks would take.  A row
 // with an infinite or NaN right-hand side counts as coupled, so that such a
 // value spreads over its line as a full solve spreads it.
+// What is left out: corrections (in the adjoint, values) further from their
+// source than the steps that were taken reach, which are below 2^-48 (2^-96) of a
+// neighbour chunk's, come out as zero or as their own row's part.  The steps go
+// on until the last row of the wavefront (X and Y: work-group) is decoupled, so such
+// values, and the last bits of values next to ones 2^23 (2^42) times as large, can
+// depend on which lines share it.  The errors against 64 bits are those of the
+// full reduction on every workload measured (FP32 2e-7 to 3e-6, its adjoint 2.4e-5,
+// FP64 4e-15).
 template <class T>
 __device__ __forceinline__ bool decoupled(const T* A, const T* C, const T* D) {
     constexpr T tiny = sizeof(T) == 4 ? (T)0x1p-48 : (T)0x1p-96;

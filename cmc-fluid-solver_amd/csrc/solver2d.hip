@@ -403,8 +403,9 @@ __global__ void __launch_bounds__(kSweepLdsThreads) k2_sweep_lds(
 // time, so it ends whatever the rows (infinite and NaN values too).  Back
 // substitution likewise from the line's end (`wb` rows early).
 // k2_sweep_lds is a chain of two FP64 divisions per row, some 220 ns each: lines
-// of 256 rows took 58 us there and of 128 rows 31, and take 18 and 14 here (build
-// of the rows 3 to 6, elimination 2 to 6, back substitution 1 to 4 us).
+// of 256 rows took 58 us there and of 128 rows 31, and take 18.7 and 14.6 here (the
+// slowest work-groups end after 15.1 and 13.3: their rows built in 6.4, elimination 6.1
+// and 4.1, back substitution 3.9 and 2.3, results 1.5; the rest is launch and drain).
 constexpr int kChunkExact = 12;
 constexpr int kChunkMaxRows = 64 * 8;   // rows of a line at most
 constexpr int kChunkMaxSystems = 2048;  // of one sweep at most: more of them fill the chip line by line
@@ -816,24 +817,6 @@ __device__ inline ErrFold fold_cat(ErrFold a, ErrFold b) {
     if (b.kind == 0) return a;
     if (a.kind == 0 || b.kind == 2) return b;
     return ErrFold{a.kind, a.ge | b.ge};
-}
-
-// Ordered fold over the work-group (thread order), result in thread 0.
-__device__ ErrFold fold_block(ErrFold s, ErrFold* sh) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-    for (int off = 1; off < 64; off <<= 1) {
-        ErrFold o;
-        o.kind = __shfl_down(s.kind, off);
-        o.ge = __shfl_down(s.ge, off);
-        if (lane + off < 64) s = fold_cat(s, o);
-    }
-    if (lane == 0) sh[wave] = s;
-    __syncthreads();
-    ErrFold r{0, 0};
-    if (threadIdx.x == 0)
-        for (int k = 0; k < nw; k++) r = fold_cat(r, sh[k]);
-    __syncthreads();
-    return r;
 }
 
 // Cell flags of the relaxation: kind in bits 0-1 (0 outside, 1 NODE_IN, 2
