@@ -37,6 +37,7 @@ from __future__ import annotations
 import argparse
 import json
 import os
+import re
 import sys
 import time
 
@@ -502,16 +503,20 @@ def stable2d_workload(steps: int = 2):
     }
 
 
-def measured_traffic(size: int, path: str):
-    """HBM bytes per sweep launch from the committed PMC summary of this
-    workload (FETCH_SIZE and WRITE_SIZE runs, scaled by a plain copy), or None."""
+def measured_traffic(size: int, path: str, variants):
+    """HBM bytes per sweep launch, the mean over X, Y and Z sweeps in these tile
+    variants, from the committed PMC summary of this workload (FETCH_SIZE and
+    WRITE_SIZE runs, scaled by a plain copy), or None."""
     fn = os.path.join(ROOT, "profiles", "pmc_sweeps_ellipsoids256_fp32.md")
     if size != 256 or path != "fused" or not os.path.exists(fn):
         return None
+    found = {}
     for line in open(fn):
-        if line.startswith("traffic_bytes_per_sweep_launch:"):
-            return float(line.split(":")[1])
-    return None
+        m = re.match(r"\s+traffic_bytes_per_sweep_launch ([XYZ]) (\d+): (\d+)", line)
+        if m:
+            found[m.group(1), int(m.group(2))] = float(m.group(3))
+    each = [found.get(k) for k in zip("XYZ", variants)]
+    return None if None in each else sum(each) / 3
 
 
 def _cpu_model() -> str:
@@ -718,7 +723,7 @@ def main():
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS,
-            "traffic": measured_traffic(args.size, head_path),
+            "traffic": measured_traffic(args.size, head_path, head["variants"]),
             "traffic_source": "profiles/pmc_sweeps_ellipsoids256_fp32.md",
             "kernel": "sweep",
             "bytes_per_step": head["sweep_bytes_per_step"],
