@@ -1095,7 +1095,7 @@ __device__ __forceinline__ bool change_divided(double qn, double qo, double tol,
 
 template <class T, int MW>
 __global__ void __launch_bounds__(1024) k2s_poisson_lds(
-    int nx, int P, int rp, int D, int bw, int cpad, const uint2* __restrict__ blist,
+    int nx, int ny, int P, int rp, int D, int bw, int cpad, const uint2* __restrict__ blist,
     const double* __restrict__ dvs, T* __restrict__ qgrid, T* __restrict__ save, double dx2,
     double dy2, double rcp, double tol, int max_sweeps, int resume, int32_t* __restrict__ status) {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -1131,9 +1131,10 @@ __global__ void __launch_bounds__(1024) k2s_poisson_lds(
         for (int c = threadIdx.x; c < 2 * kPoisGroup; c += blockDim.x) fold[c] = 0;
         if (threadIdx.x == 0) s_first = g;
         __syncthreads();
-        // to the end of sweep g - 1: its start, rows, columns and the inner
-        // front's two steps, in whole turns of the loops' four steps
-        const int steps = (((g - 1) / D) * P + ((g - 1) % D) * kPoisLag + nx + P + 2 + 3) & ~3;
+        // to the end of sweep g - 1: its start, rows, columns (x = 1 .. ny, not the whole
+        // turn of P: of 12 x 10 cells 11 steps, not 60) and the inner front's two
+        // steps, in whole turns of the loops' four steps
+        const int steps = (((g - 1) / D) * P + ((g - 1) % D) * kPoisLag + nx + ny + 1 + 2 + 3) & ~3;
         if (inner) {
             // Branch-free but for the rare cases (a change too close to tol to
             // tell, the end of a turn), each tested once for the MW cells.
@@ -1968,7 +1969,7 @@ class Solver2D final : public ISolver2 {
             if (fronts) {
                 auto kern = rl_mw == 2 ? k2s_poisson_lds<T, 2> : k2s_poisson_lds<T, 1>;
                 hipLaunchKernelGGL(kern, dim3(1), dim3(rl_D / rl_mw * rl_rp + 64 * rl_bw),
-                                   sizeof(T) * (size_t)(nx + 2) * rl_P, st, nx, rl_P, rl_rp, rl_D, rl_bw,
+                                   sizeof(T) * (size_t)(nx + 2) * rl_P, st, nx, ny, rl_P, rl_rp, rl_D, rl_bw,
                                    rl_cpad, d_blist, d_dvs, d_qpad, d_qsave, dx2, dy2, rcp, ptol, chunk,
                                    resume, d_pstat);
                 CMCX_LAUNCH_CHECK();
